@@ -1,0 +1,664 @@
+// Extend (chunked prefill) attention kernels and entry points.
+#include "mkv_attn.h"
+
+namespace mkv {
+
+// The extend kernel's one-head tiles (rows of 2 * head_dim bytes) take a
+// swizzle per tile, each measured free of bank conflicts at head_dim 64, 128
+// and 256 (no single row swizzle is, for both reads, at all three):
+//   K tile: chunk c of row r at c ^ r          (ds_read_b128 reads)
+//   V tile: chunk c of row r at c ^ v_swz(r)   (ds_read_b64_tr_b16 reads),
+// v_swz linear over GF(2) in the row's four bits, which flip chunk bits by
+// 2, 4, 11 and 1. With the decode swizzle above both reads were 2-way
+// conflicted at head_dim 128 (47% of the kernel's LDS cycles stalled).
+__device__ __forceinline__ int ext_k_swz(int row, int cpr) { return row & (cpr - 1); }
+__device__ __forceinline__ int ext_v_swz(int row, int cpr) {
+  const int s = ((row & 1) << 1) ^ ((row & 2) << 1) ^ (((row >> 2) & 1) * 11) ^ ((row >> 3) & 1);
+  return s & (cpr - 1);
+}
+
+// ===========================================================================
+// Extend (chunked prefill) attention: causal attention of each sequence's
+// newest q_len tokens over its whole cache (the chunk's own K/V already
+// appended), the seq_q > 1 path of inference-model-qwen/src/model.rs:410-416
+// with the causal mask of model.rs:542-555 (a key at position j is visible to
+// the query at position p iff j <= p).
+//
+// One workgroup per (query tile of 16 or 32 positions, KV head, sequence,
+// key-range split); per 16-position sub-tile, W/TP >= G waves, wave g
+// computing query head h*G + g for the sub-tile's positions (the MFMA column
+// dimension). The workgroup streams the head's K/V blocks 0..(last tile
+// position)/16 (its split's share of them) through a double-buffered LDS
+// tile (rows of one head: D*2 bytes; K and V tiles each with their own
+// bank-conflict-free swizzle), loaded cooperatively one step of two blocks
+// ahead; scores, online softmax and the V^T transpose reads follow the
+// decode kernel, with the causal mask applied on blocks that reach past a
+// sub-tile's first position. Steps whose keys every query of the workgroup
+// sees (all but the last one or two of a tile) run a lean form: block ids
+// staged in LDS and checked once, wave-uniform load bases, no masks, and the
+// PV product on one full-rate 16x16x32 MFMA per 16 dims over both blocks.
+// ===========================================================================
+
+// Extend kernel: two blocks (32 keys) per softmax step, steps loaded one
+// ahead (two blocks in flight). Measured against one block per step with a
+// 4-step ring: equal at head_dim 128, 3.5% faster at 256; four blocks per
+// step raise the register count past two workgroups per CU.
+constexpr int kExtKB = 2;  // blocks per softmax step of the extend kernel
+constexpr int kExtR = 2;   // ring depth (steps) of the extend kernel
+// Block ids a workgroup stages in LDS for its unmasked steps (16k keys);
+// a longer key range takes the scalar table reads throughout.
+constexpr int kExtIdCap = 1024;
+
+// Workgroups are dealt to the 8 XCDs round-robin by linear index. The
+// launch has 8 * per_xcd workgroups; workgroup L becomes logical index
+// (L % 8) * per_xcd + L / 8, so each XCD receives a contiguous run of
+// logical indices: the query tiles of one (sequence, KV head) share that
+// XCD's L2 while they stream the same K/V. Logical index = (tiles - 1 -
+// tile) + tiles * (group + hgroups * (head + Hkv * (sequence + B * split)));
+// false for the padding past the last one. `h` returns head * hgroups +
+// group. The last tile of a chunk attends the most keys,
+// so a sequence's tiles start longest first (causal 2k-token prompts: 518 ->
+// 487 us), leaving the short ones for the tail.
+__device__ __forceinline__ bool ext_tile(const ExtArgs &e, int Hkv, int &t, int &h, int &b, int &sp) {
+  const int L = blockIdx.x;
+  const int logical = (L & 7) * e.per_xcd + (L >> 3);
+  const int heads = Hkv * e.hgroups;
+  const int per_split = e.tiles * heads * e.B;
+  if (logical >= per_split * e.splits) return false;
+  const int r = logical % per_split;
+  sp = logical / per_split;
+  t = e.tiles - 1 - r % e.tiles;
+  h = (r / e.tiles) % heads;
+  b = r / (e.tiles * heads);
+  return true;
+}
+
+template <int D, int W, int KB, int R, int TP>
+__global__ void __launch_bounds__(64 * W) attn_extend_kernel(KArgs a, ExtArgs e) {
+  constexpr int NR = D / 32, NT = D / 16;
+  constexpr int RB = D * 2;                           // LDS tile row: one head's K or V row
+  constexpr int CPR = RB / 16;                        // 16-byte chunks per tile row
+  constexpr int TILE = 16 * RB;
+  constexpr int BCH = 2 * 16 * CPR;                   // chunks of K + V of one block
+  constexpr int NCH = KB * BCH;                       // chunks of one step (KB blocks)
+  constexpr int LPL = (NCH + 64 * W - 1) / (64 * W);  // loads per lane per step
+  static_assert(R % 2 == 0, "even ring: stage s of an unrolled round uses LDS buffer s & 1");
+  constexpr int WG = W / TP;                          // waves per 16-position sub-tile
+  static_assert(W % TP == 0, "whole sub-tiles per workgroup");
+  __shared__ __attribute__((aligned(16))) uint8_t tiles[2][KB][2][TILE];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m16 = lane & 15, g4 = lane >> 4, a4 = m16 >> 2, rq = m16 & 3;
+  int t, hx, b, sp;
+  if (!ext_tile(e, a.Hkv, t, hx, b, sp)) return;
+  const int h = hx / e.hgroups, hg = hx % e.hgroups;  // KV head; group of W / TP query heads
+  const bool virt = e.q_indptr == nullptr;  // one sequence; the host checked its table length
+  const int q0 = virt ? 0 : e.q_indptr[b], nq = virt ? e.v_nq : e.q_indptr[b + 1] - q0;
+  if (nq <= 0 || 16 * TP * t >= nq) return;
+  const int ctx = virt ? e.v_ctx : e.ctx[b];
+  // (With partials, a chunk longer than max_q_len or a q_indptr past
+  // num_seqs * max_q_len tokens would address partial rows past the workspace.)
+  if ((e.causal && nq > ctx) || ctx < 1 || ctx > e.max_ctx ||
+      ((e.splits > 1 || e.partial) && (nq > e.max_q || q0 < 0 || (int64_t)q0 + nq > (int64_t)e.B * e.max_q))) {
+    if (threadIdx.x == 0 && t == 0) record_error(a.d_err, MKV_DEVERR_CTX);
+    return;
+  }
+  const int tab0 = virt ? 0 : a.indptr[b], nbt = (ctx + kPageSize - 1) / kPageSize;
+  if (!virt && (tab0 < 0 || a.indptr[b + 1] - tab0 < nbt)) {
+    if (threadIdx.x == 0 && t == 0) record_error(a.d_err, MKV_DEVERR_TABLE);
+    return;
+  }
+  // The table is read through the constant address space: scalar loads,
+  // whose wait does not drain the vector-load ring (a vector load of a block
+  // id needs vmcnt(0) before its readfirstlane).
+  typedef const __attribute__((address_space(4))) int32_t const_i32;
+  const const_i32 *table = (const const_i32 *)(a.ids + tab0);
+  // The workgroup holds TP sub-tiles of 16 positions; wave = (sub-tile, head slot).
+  const int sub = wave / WG, hw = wave % WG;
+  const int row0 = 16 * (TP * t + sub);                  // first chunk row of this wave's sub-tile
+  // Its first query position; without the causal mask every query stands at
+  // the last position and sees all ctx keys.
+  const int qlo = e.causal ? ctx - nq + row0 : ctx - 1;
+  const int qhi_wg = e.causal ? min(ctx - nq + 16 * TP * (t + 1) - 1, ctx - 1) : ctx - 1;
+  const int n = qhi_wg / kPageSize + 1;                  // blocks the workgroup streams: keys 0..qhi_wg
+  const int nw = min(n, (qlo + 15) / kPageSize + 1);     // blocks this wave's sub-tile sees
+  // Steps of KB blocks; with splits, this workgroup takes its share of them
+  // (a short context can leave a split none: it stores an empty partial).
+  const int nsteps_all = (n + KB - 1) / KB;
+  const int sps = (nsteps_all + e.splits - 1) / e.splits;
+  const int st0 = min(sp * sps, nsteps_all), st1 = min(st0 + sps, nsteps_all);
+  const int hslot = hg * WG + hw;  // this wave's query head among the KV head's G
+  const bool computes = hslot < a.G;
+  const int hq = h * a.G + min(hslot, a.G - 1);
+  const int qp = e.causal ? qlo + m16 : ctx - 1;  // this lane's query position (rows past nq: unused)
+  const int64_t spare = dummy_offset(a);
+
+  // Q^T operand: lane holds Q[row 16t + lane%16][32r + 8*(lane/16) .. +8].
+  bf16x8 qop[NR];
+  {
+    const int row = min(row0 + m16, nq - 1);
+    const uint8_t *qp8 = static_cast<const uint8_t *>(a.q) + ((int64_t)(q0 + row) * a.Hq + hq) * D * 2;
+#pragma unroll
+    for (int r = 0; r < NR; r++)
+      qop[r] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(qp8 + 2 * (32 * r + 8 * g4)));
+  }
+
+  // Ring slot of one step: lane loads chunks c = threadIdx.x + 64*W*i of the
+  // step's KB blocks (block kb = c / BCH: K rows then V rows of head h).
+  // Blocks past n and chunks past the step read 128 bytes of a block picked
+  // by the workgroup index, so every stage issues the same loads.
+  u32x4 ring[R][LPL];
+  uint32_t badr[R];  // bit kb: block kb of the step was rejected
+  auto issue = [&](u32x4 (&d)[LPL], uint32_t &bad, int step) {
+    int32_t blk[KB];
+    bad = 0;
+#pragma unroll
+    for (int kb = 0; kb < KB; kb++) {
+      const int k = step * KB + kb;
+      blk[kb] = k < n ? table[k] : 0;  // uniform: a scalar load
+      if (k < n && (blk[kb] < 0 || blk[kb] >= a.nblocks)) {
+        bad |= 1u << kb;
+        blk[kb] = 0;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < LPL; i++) {
+      const int c = (int)threadIdx.x + 64 * W * i;
+      const int kb = min(c / BCH, KB - 1), rem = c % BCH;
+      const int kv = rem / (16 * CPR), rem2 = rem % (16 * CPR), row = rem2 / CPR, cc = rem2 % CPR;
+      int32_t bk = blk[0];
+#pragma unroll
+      for (int j = 1; j < KB; j++) bk = kb == j ? blk[j] : bk;
+      const bool real = c < NCH && step * KB + kb < n;
+      const uint8_t *plane = kv ? a.v_plane : a.k_plane;
+      const int64_t off = real ? (int64_t)bk * a.block_bytes + (int64_t)row * a.row_bytes + h * RB + 16 * cc
+                               : spare + 16 * (lane & 7);
+      d[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>((real ? plane : a.k_plane) + off));
+    }
+  };
+
+  // Unmasked steps take a lean path. The ids of the workgroup's blocks
+  // [kfirst, kend) are staged in LDS and range-checked once (any rejected id:
+  // the generic path throughout, which masks it and records the error).
+  // Chunk c = 64 * (wave + W * i) + lane of a step lies in one (block, K/V)
+  // plane per wave, so a load is a wave-uniform base (block id, plane) plus a
+  // lane offset (row, chunk, head) fixed for the whole launch.
+  // (More than four loads per lane and step would hold more registers than the
+  // lean path saves: those launches keep the generic path.)
+  constexpr bool kLean = LPL <= 4;
+  __shared__ int32_t ids_s[kLean ? kExtIdCap : 1];
+  const int kfirst = st0 * KB, kend = min(st1 * KB, n);
+  int fast = kLean && kend - kfirst <= kExtIdCap;
+  if (fast) {
+    int badl = 0;
+    const int32_t *tg = a.ids + tab0 + kfirst;
+    for (int i = (int)threadIdx.x; i < kend - kfirst; i += 64 * W) {
+      const int32_t id = tg[i];
+      badl |= (id < 0) | (id >= a.nblocks);
+      ids_s[i] = id;
+    }
+    fast = !__syncthreads_or(badl);
+  }
+  fast = __builtin_amdgcn_readfirstlane(fast);
+  // A wave past the step's chunks (head_dim 64 with 16 waves) loads the
+  // step's last chunks again and does not store them: one load form, so the
+  // compiler's in-order load counting stays exact.
+  constexpr bool kAllVal = NCH % (64 * W) == 0;
+  uint32_t flo[LPL], fwr[LPL];  // lane offset in the block; LDS offset in one ring buffer
+  int fkb[LPL];                 // wave-uniform block of the step
+  const uint8_t *fpl[LPL];      // wave-uniform plane (K or V)
+  bool fval[LPL];               // wave-uniform: the wave's chunk is stored
+#pragma unroll
+  for (int i = 0; i < LPL; i++) {
+    const int cw = 64 * (wave + W * i);
+    fval[i] = kAllVal || cw < NCH;
+    const int cu = min(cw, NCH - 64);
+    const int pl = cu / (16 * CPR), kv = pl & 1;
+    fkb[i] = pl >> 1;
+    fpl[i] = kv ? a.v_plane : a.k_plane;
+    const int rem2 = cu % (16 * CPR) + lane, row = rem2 / CPR, cc = rem2 % CPR;
+    flo[i] = (uint32_t)(row * (int)a.row_bytes + h * RB + 16 * cc);
+    fwr[i] = (uint32_t)((2 * fkb[i] + kv) * TILE + row * RB + ((cc ^ (kv ? ext_v_swz(row, CPR) : ext_k_swz(row, CPR))) << 4));
+  }
+  // A step whose KB blocks all lie in [kfirst, kend).
+  auto issue_fast = [&](u32x4 (&d)[LPL], uint32_t &bad, int step) {
+    bad = 0;
+#pragma unroll
+    for (int i = 0; i < LPL; i++) {
+      const int32_t bk = __builtin_amdgcn_readfirstlane(ids_s[step * KB + fkb[i] - kfirst]);
+      d[i] = __builtin_nontemporal_load(
+          reinterpret_cast<const u32x4 *>(fpl[i] + (int64_t)bk * a.block_bytes + flo[i]));
+    }
+  };
+
+  MStateT<D> st;
+#pragma unroll
+  for (int nn = 0; nn < NT; nn++) st.O[nn] = f32x4{0.f, 0.f, 0.f, 0.f};
+  st.m = -INFINITY;
+  st.l = 0.0f;
+  const float inv_sl2 = 1.0f / a.sl2;
+  float thr = -INFINITY;  // raw-score rescale threshold
+  int k_rd[NR], v_rd[NT];
+  const int vrow = 4 * g4 + a4;
+#pragma unroll
+  for (int r = 0; r < NR; r++) k_rd[r] = m16 * RB + (((g4 + 4 * r) ^ ext_k_swz(m16, CPR)) << 4);
+#pragma unroll
+  for (int nn = 0; nn < NT; nn++)
+    v_rd[nn] = vrow * RB + (((2 * nn + (rq >> 1)) ^ ext_v_swz(vrow, CPR)) << 4) + 8 * (rq & 1);
+
+  // FAST: every block of the step is in range and fully visible to every
+  // query of the workgroup (no mask), and the step issued R - 1 ahead lies
+  // in the staged ids.
+  auto stage = [&](auto fast_c, int s, int step) {
+    constexpr bool FAST = decltype(fast_c)::value;
+    if constexpr (FAST) issue_fast(ring[(s + R - 1) % R], badr[(s + R - 1) % R], step + R - 1);
+    else issue(ring[(s + R - 1) % R], badr[(s + R - 1) % R], step + R - 1);
+    // step = (multiple of R) + s: buffer s & 1 alternates like step & 1 and
+    // is a compile-time constant here (immediate LDS offsets).
+#pragma unroll
+    for (int i = 0; i < LPL; i++) {
+      if constexpr (FAST) {
+        if (kAllVal || fval[i]) *reinterpret_cast<u32x4 *>(&tiles[s & 1][0][0][0] + fwr[i]) = ring[s][i];
+        continue;
+      }
+      const int c = (int)threadIdx.x + 64 * W * i;
+      if (c < NCH) {
+        const int kb = c / BCH, rem = c % BCH;
+        const int kv = rem / (16 * CPR), rem2 = rem % (16 * CPR), row = rem2 / CPR, cc = rem2 % CPR;
+        // V rows past the context or of a rejected block are stored as
+        // zeros (stale slots may hold any bit pattern, and p = 0 times NaN
+        // would poison O); K rows there are masked in the scores instead.
+        u32x4 val = ring[s][i];
+        if (kv && (((badr[s] >> kb) & 1) || kPageSize * (step * KB + kb) + row >= ctx)) val = u32x4{0u, 0u, 0u, 0u};
+        *reinterpret_cast<u32x4 *>(tiles[s & 1][kb][kv] + row * RB + ((cc ^ (kv ? ext_v_swz(row, CPR) : ext_k_swz(row, CPR))) << 4)) = val;
+      }
+    }
+    __syncthreads();
+    if (!computes) return;
+    const uint32_t bad = FAST ? 0u : badr[s];
+    if (!FAST && bad && lane == 0) record_error(a.d_err, MKV_DEVERR_BLOCK);
+    // Raw scores of the step's blocks (masked ones -inf). Lane holds
+    // sr[kb][i] = S[key 16k + 4*g4 + i][query position qlo + lane%16].
+    float sr[KB][4];
+    float mloc = -INFINITY;
+    bool masked = false;  // some block of the step needs the causal / context mask (uniform)
+#pragma unroll
+    for (int kb = 0; kb < KB; kb++) {
+      const int k = step * KB + kb;
+      if (!FAST && k >= nw) {  // uniform: past this sub-tile's last position (or past n in the last step)
+#pragma unroll
+        for (int i = 0; i < 4; i++) sr[kb][i] = -INFINITY;
+        masked = true;
+        continue;
+      }
+      const uint8_t *tk = tiles[s & 1][kb][0];
+      u32x4 kq[NR];
+#pragma unroll
+      for (int r = 0; r < NR; r++) kq[r] = *reinterpret_cast<const u32x4 *>(tk + k_rd[r]);
+      f32x4 S = {0.f, 0.f, 0.f, 0.f};
+      // Where one workgroup fills a CU (two sub-tiles, or head_dim 256 with
+      // 8 or more waves) the score MFMAs issue at raised wave priority, so a
+      // wave that reaches them overtakes the waves busy with exponentials
+      // and the matrix pipe stays fed (8 x 512 after 4k: 455 -> 435-445 us at priority 1, about
+      // 1% more at 3; head_dim 256: 259 -> 255 us). The same around the PV
+      // products or the load issue gained nothing, and with one sub-tile at
+      // head_dim <= 128 (two workgroups per CU) it cost 16-token chunks 15%.
+      constexpr bool kPrio = TP == 2 || (D == 256 && W >= 8);
+      if constexpr (kPrio) __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+      for (int r = 0; r < NR; r++)
+        S = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kq[r]), qop[r], S, 0, 0, 0);
+      if constexpr (kPrio) __builtin_amdgcn_s_setprio(0);
+      const bool kbad = (bad >> kb) & 1;
+      const bool full = FAST || (!kbad && kPageSize * k + kPageSize - 1 <= qlo && kPageSize * k + kPageSize <= ctx);
+#pragma unroll
+      for (int i = 0; i < 4; i++) sr[kb][i] = S[i];
+      if (!full) {  // only the last blocks of a tile (and rejected ones)
+        masked = true;
+        const int kp0 = kPageSize * k + 4 * g4;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (kbad || kp0 + i > qp || kp0 + i >= ctx) sr[kb][i] = -INFINITY;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++) mloc = fmaxf(mloc, sr[kb][i]);
+    }
+    // Rescale only when some score passes the running max by the slack
+    // (st.m in scaled log2 units, thr = (st.m + slack) / (scale * log2 e) in
+    // raw ones): checked on the lane's own scores first, so the column-wide
+    // max (two cross-lane steps) runs only on the rare steps that need it.
+    if (__ballot(mloc > thr)) {
+      mloc = fmaxf(mloc, __shfl_xor(mloc, 16));
+      mloc = fmaxf(mloc, __shfl_xor(mloc, 32));
+      const float ms = mloc * a.sl2;
+      const bool need = ms > st.m + kRescaleSlack;
+      const float mn = need ? ms : st.m;
+      // A column with nothing visible yet (possible in a later key range)
+      // keeps m = -inf, l = 0, O = 0: scale 0, not exp2(-inf - -inf) = NaN.
+      const float al = st.m == -INFINITY ? 0.0f : fast_exp2(st.m - mn);
+      st.l *= al;
+#pragma unroll
+      for (int nn = 0; nn < NT; nn++) st.O[nn] *= al;
+      st.m = mn;
+      thr = (mn + kRescaleSlack) * inv_sl2;
+    }
+    if constexpr (FAST && KB == 2) {
+      // Both blocks in one full-rate 16x16x32 product per 16 dims: lane
+      // group g4's k-slots 0-3 are keys 4*g4..+3 of the first block and 4-7
+      // the same keys of the second, in P^T (the score layout) and in V^T
+      // (one transposed read per block).
+      uint32_t pk[4];
+#pragma unroll
+      for (int kb = 0; kb < 2; kb++) {
+        float pr[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) pr[i] = fast_exp2(fmaf(sr[kb][i], a.sl2, -st.m));
+        st.l += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+        pk[2 * kb] = pack_bf16x2(pr[0], pr[1]);
+        pk[2 * kb + 1] = pack_bf16x2(pr[2], pr[3]);
+      }
+      const bf16x8 pb = __builtin_bit_cast(bf16x8, u32x4{pk[0], pk[1], pk[2], pk[3]});
+      const uint8_t *tv0 = tiles[s & 1][0][1], *tv1 = tiles[s & 1][1][1];
+#pragma unroll
+      for (int nn = 0; nn < NT; nn++) {
+        const i16x4s r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(tv0 + v_rd[nn]));
+        const i16x4s r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(tv1 + v_rd[nn]));
+        const uint64_t w0 = __builtin_bit_cast(uint64_t, r0), w1 = __builtin_bit_cast(uint64_t, r1);
+        const bf16x8 va = __builtin_bit_cast(bf16x8, u32x4{(uint32_t)w0, (uint32_t)(w0 >> 32), (uint32_t)w1,
+                                                            (uint32_t)(w1 >> 32)});
+        st.O[nn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb, st.O[nn], 0, 0, 0);
+      }
+      return;
+    }
+#pragma unroll
+    for (int kb = 0; kb < KB; kb++) {
+      const int k = step * KB + kb;
+      if (!FAST && k >= nw) continue;  // uniform
+      float pr[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) pr[i] = fast_exp2(fmaf(sr[kb][i], a.sl2, -st.m));
+      if (!FAST && masked) {  // a fully masked column has m = -inf: keep its p at 0, not NaN
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (sr[kb][i] == -INFINITY) pr[i] = 0.0f;
+      }
+      st.l += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+      const uint32_t p01 = pack_bf16x2(pr[0], pr[1]), p23 = pack_bf16x2(pr[2], pr[3]);
+      const i16x4 pb = __builtin_bit_cast(i16x4, (uint64_t)p01 | ((uint64_t)p23 << 32));
+      // O^T += V^T . P^T (V rows past the context were zeroed in LDS;
+      // causally hidden rows have p = 0).
+      const uint8_t *tv = tiles[s & 1][kb][1];
+#pragma unroll
+      for (int nn = 0; nn < NT; nn++) {
+        const i16x4s raw = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(tv + v_rd[nn]));
+        st.O[nn] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(i16x4, raw), pb, st.O[nn], 0, 0, 0);
+      }
+    }
+  };
+
+#pragma unroll
+  for (int s = 0; s < R - 1; s++) issue(ring[s], badr[s], st0 + s);
+  // Fast steps: [st0, fast_end), blocks below the workgroup's first query
+  // position and below ctx (all keys visible to all its queries), with the
+  // steps issued R - 1 ahead inside [kfirst, kend).
+  const int fb = e.causal ? min((ctx - nq + 16 * TP * t + 1) / kPageSize, ctx / kPageSize) : ctx / kPageSize;
+  const int fast_end = fast ? max(st0, min(min(st1, fb / KB), kend / KB - (R - 1))) : st0;
+  const std::integral_constant<bool, true> kFast;
+  const std::integral_constant<bool, false> kGeneric;
+  int k0 = st0;
+  for (int it = 0, nit = (fast_end - st0) / R; it < nit; it++, k0 += R) {
+#pragma unroll
+    for (int s = 0; s < R; s++) stage(kFast, s, k0 + s);
+  }
+  for (int it = 0, nit = (st1 - k0) / R; it < nit; it++, k0 += R) {
+#pragma unroll
+    for (int s = 0; s < R; s++) stage(kGeneric, s, k0 + s);
+  }
+#pragma unroll
+  for (int s = 0; s < R - 1; s++)
+    if (k0 + s < st1) stage(kGeneric, s, k0 + s);
+
+  if (!computes) return;
+  st.l += __shfl_xor(st.l, 16);
+  st.l += __shfl_xor(st.l, 32);
+  const int row = row0 + m16;
+  if (row >= nq) return;
+  if (e.splits > 1 || e.partial) {  // f32 partial (m, l, O) of this key range, merged later
+    const int64_t prow = ((int64_t)(q0 + row) * a.Hq + hq) * e.splits + sp;
+    float *wo = a.ws_o + prow * D + 4 * g4;
+#pragma unroll
+    for (int nn = 0; nn < NT; nn++) *reinterpret_cast<f32x4 *>(wo + 16 * nn) = st.O[nn];
+    if (g4 == 0) *reinterpret_cast<float2 *>(a.ws_ml + 2 * prow) = make_float2(st.m, st.l);
+    return;
+  }
+  const float f = final_scale(st.m, st.l, a.zero_sink);
+  uint16_t *op = reinterpret_cast<uint16_t *>(a.o) + ((int64_t)(q0 + row) * a.Hq + hq) * D + 4 * g4;
+#pragma unroll
+  for (int nn = 0; nn < NT; nn++)
+    *reinterpret_cast<uint2 *>(op + 16 * nn) = make_uint2(pack_bf16x2(st.O[nn][0] * f, st.O[nn][1] * f),
+                                                          pack_bf16x2(st.O[nn][2] * f, st.O[nn][3] * f));
+}
+
+// Log-sum-exp merge of the extend kernel's key-range partials: one wave per
+// (query token, query head) row, partials row * splits + s.
+template <int D, bool BF16>
+__global__ void __launch_bounds__(256) merge_ext_kernel(KArgs a, ExtArgs e) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t row = (int64_t)blockIdx.x * 4 + wave;
+  const int64_t tokens = min((int64_t)e.q_indptr[e.B], (int64_t)e.B * e.max_q);
+  if (row >= tokens * a.Hq) return;
+  merge_rows<D, BF16>(a, lane, row * e.splits, 1, e.splits, row);
+}
+
+}  // namespace mkv
+
+using namespace mkv;
+
+extern "C" int mkv_extend_attention(mkv_pool *pool, int32_t layer, const void *d_q, void *d_o,
+                                    const int32_t *d_q_indptr, const int32_t *d_block_indptr,
+                                    const int32_t *d_block_ids, const int32_t *d_ctx_lens, int32_t num_seqs,
+                                    int32_t max_q_len, int32_t max_ctx_len, float scale, uint32_t flags,
+                                    void *stream) {
+  if (!pool) return set_error(MKV_ERR_INVALID_ARGUMENT, "NULL pool");
+  Pool *p = reinterpret_cast<Pool *>(pool);
+  const Geom &g = p->g;
+  bool use_mfma = false;
+  int rc = check_common(p, layer, flags, scale, use_mfma);
+  if (rc) return rc;
+  if (!d_q || !d_o || !d_q_indptr || !d_block_indptr || !d_block_ids || !d_ctx_lens)
+    return set_error(MKV_ERR_INVALID_ARGUMENT, "NULL device pointer");
+  if (num_seqs < 0 || max_q_len < 0 || max_ctx_len < 0)
+    return set_error(MKV_ERR_INVALID_ARGUMENT, "negative sizes");
+  if (num_seqs == 0 || max_q_len == 0) return MKV_OK;
+  if (max_q_len > max_ctx_len)
+    return set_error(MKV_ERR_INVALID_ARGUMENT, "max_q_len %d > max_ctx_len %d", max_q_len, max_ctx_len);
+  const int G = g.Hq / g.Hkv;
+  if (!aligned16(d_q) || !aligned16(d_o)) return set_error(MKV_ERR_INVALID_ARGUMENT, "q and o must be 16-byte aligned");
+  DeviceGuard guard(p->device);
+  hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+  if (!use_mfma || G > 16) {  // per-token segments on the decode kernels
+    KArgs a = make_kargs(p, layer, d_q, d_o, d_block_indptr, d_block_ids, scale, flags, use_mfma);
+    return launch_ext_segments(p, a, d_q_indptr, d_ctx_lens, num_seqs, max_q_len, max_ctx_len, use_mfma, hs);
+  }
+  KArgs a = make_kargs(p, layer, d_q, d_o, d_block_indptr, d_block_ids, scale, flags, true);
+  ExtArgs e{};
+  e.q_indptr = d_q_indptr;
+  e.ctx = d_ctx_lens;
+  e.B = num_seqs;
+  e.max_ctx = max_ctx_len;
+  e.max_q = max_q_len;
+  e.causal = 1;
+  return launch_ext_tiles(p, a, e, 4, hs);
+}
+
+extern "C" int mkv_extend_attention_host(mkv_pool *pool, int32_t layer, const void *d_q, void *d_o,
+                                         const int32_t *h_q_lens, const int32_t *h_ctx_lens,
+                                         const uint32_t *h_block_indptr, const uint32_t *h_block_ids,
+                                         int32_t num_seqs, float scale, uint32_t flags, void *stream) {
+  if (!pool) return set_error(MKV_ERR_INVALID_ARGUMENT, "NULL pool");
+  Pool *p = reinterpret_cast<Pool *>(pool);
+  if (num_seqs < 0) return set_error(MKV_ERR_INVALID_ARGUMENT, "num_seqs < 0");
+  if (num_seqs == 0) return MKV_OK;
+  if (!h_q_lens) return set_error(MKV_ERR_INVALID_ARGUMENT, "NULL q_lens");
+  int32_t max_ctx = 0;
+  int rc = check_host_tables(p->g, h_block_indptr, h_block_ids, h_ctx_lens, num_seqs, &max_ctx);
+  if (rc) return rc;
+  int32_t max_q = 0;
+  int64_t rows = 0;
+  for (int32_t b = 0; b < num_seqs; b++) {
+    if (h_q_lens[b] < 0 || h_q_lens[b] > h_ctx_lens[b])
+      return set_error(MKV_ERR_INVALID_ARGUMENT, "sequence %d: %d new tokens outside [0, ctx %d]", b, h_q_lens[b],
+                       h_ctx_lens[b]);
+    max_q = std::max(max_q, h_q_lens[b]);
+    rows += h_q_lens[b];
+  }
+  if (rows > INT32_MAX) return set_error(MKV_ERR_INVALID_ARGUMENT, "more than 2^31 - 1 query rows");
+  if (max_q == 0) return MKV_OK;
+  const size_t nids = h_block_indptr[num_seqs];
+  const size_t n = 3 * (size_t)num_seqs + 2 + nids;  // q_indptr | indptr | ctx | ids
+  DeviceGuard guard(p->device);
+  hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+  // Every layer of a step passes the same chunks and tables: uploaded once
+  // per step.
+  std::vector<int32_t> &stg = p->stage_tmp;
+  stg.resize(n);
+  int32_t *qp = stg.data(), *ip = qp + num_seqs + 1, *cl = ip + num_seqs + 1, *ix = cl + num_seqs;
+  qp[0] = 0;
+  for (int32_t b = 0; b < num_seqs; b++) qp[b + 1] = qp[b] + h_q_lens[b];
+  for (int32_t b = 0; b <= num_seqs; b++) ip[b] = (int32_t)h_block_indptr[b];
+  std::memcpy(cl, h_ctx_lens, (size_t)num_seqs * 4);
+  if (nids) std::memcpy(ix, h_block_ids, nids * 4);
+  MetaSlot *sl = nullptr;
+  if ((rc = stage_cached(p, p->extend_cache, stg.data(), n, hs, &sl))) return rc;
+  const int32_t *d = sl->d;
+  rc = mkv_extend_attention(pool, layer, d_q, d_o, d, d + num_seqs + 1, d + 3 * num_seqs + 2, d + 2 * num_seqs + 2,
+                            num_seqs, max_q, max_ctx, scale, flags, stream);
+  const int rr = meta_release(sl, hs);
+  return rc ? rc : rr;
+}
+
+// The extend kernel's instantiation for head_dim D, W waves and TP
+// sub-tiles of 16 positions per workgroup.
+const void *mkv::ext_kernel(int D, int W, int TP) {
+  const void *fn = nullptr;
+#define MKV_EXT_FN(DD, TT)                                                                                  \
+  do {                                                                                                      \
+    switch (W / TT) {                                                                                       \
+      case 1: fn = reinterpret_cast<const void *>(&attn_extend_kernel<DD, 1 * TT, kExtKB, kExtR, TT>); break; \
+      case 2: fn = reinterpret_cast<const void *>(&attn_extend_kernel<DD, 2 * TT, kExtKB, kExtR, TT>); break; \
+      case 4: fn = reinterpret_cast<const void *>(&attn_extend_kernel<DD, 4 * TT, kExtKB, kExtR, TT>); break; \
+      case 8: fn = reinterpret_cast<const void *>(&attn_extend_kernel<DD, 8 * TT, kExtKB, kExtR, TT>); break; \
+      default: fn = reinterpret_cast<const void *>(&attn_extend_kernel<DD, 16, kExtKB, kExtR, 1>); break;     \
+    }                                                                                                       \
+  } while (0)
+  switch (D) {
+    case 64: if (TP == 2) MKV_EXT_FN(64, 2); else MKV_EXT_FN(64, 1); break;
+    case 128: if (TP == 2) MKV_EXT_FN(128, 2); else MKV_EXT_FN(128, 1); break;
+    default:
+      fn = W == 4 ? reinterpret_cast<const void *>(&attn_extend_kernel<256, 4, kExtKB, kExtR, 1>)
+                  : reinterpret_cast<const void *>(&attn_extend_kernel<256, 8, kExtKB, kExtR, 1>);
+      break;
+  }
+#undef MKV_EXT_FN
+  return fn;
+}
+
+// Resident workgroups per CU of an extend instantiation (occupancy query,
+// once per pool and instantiation); -1 when unknown.
+int mkv::ext_resident_per_cu(Pool *p, const void *fn, int W, int TP) {
+  const Geom &g = p->g;
+  int &per_cu = p->ext_per_cu[g.D == 64 ? 0 : g.D == 128 ? 1 : 2][W == 1 ? 0 : W == 2 ? 1 : W == 4 ? 2 : W == 8 ? 3 : 4][TP - 1];
+  if (per_cu == 0) {
+    int n_cu = 0;
+    DeviceGuard guard(p->device);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n_cu, fn, 64 * W, 0) != hipSuccess) {
+      (void)hipGetLastError();  // leave no sticky error: no splitting
+      n_cu = 0;
+    }
+    per_cu = n_cu > 0 ? n_cu : -1;
+  }
+  return per_cu;
+}
+
+// MFMA query tiles of the extend kernel for e (B, max_q, max_ctx, causal,
+// partial and the sequence arguments set): picks the instantiation and the
+// key-range split (at most split_cap), grows the pool workspace when
+// partials are stored, launches, and merges the splits unless e.partial
+// (then a.ws_ml / a.ws_o and e.splits describe the partials left). With
+// beside, the tiles share the device with a decode launch that holds one
+// workgroup per CU: one sub-tile per workgroup, and the split aims at one
+// workgroup per CU.
+int mkv::launch_ext_tiles(Pool *p, KArgs &a, ExtArgs &e, int split_cap, hipStream_t hs, bool beside) {
+  const Geom &g = p->g;
+  const int G = g.Hq / g.Hkv;
+  const int64_t num_seqs = e.B, max_q_len = e.max_q, max_ctx_len = e.max_ctx;
+  if (((max_q_len + 15) / 16 * g.Hq * num_seqs) * split_cap + 8 > INT32_MAX)
+    return set_error(MKV_ERR_INVALID_ARGUMENT, "grid too large");
+  e.splits = 1;
+  // Waves per 16-position sub-tile: the next power of two >= G. Two
+  // sub-tiles per workgroup share each K/V tile (K/V streamed once per 32
+  // positions) where that stays within 16 waves and their register budget
+  // (head_dim <= 128) and chunks are longer than one sub-tile. Measured at
+  // Qwen-7B heads: 8 x 512 after 4k 526 -> 480 us, 8 x 2,048 prompts 560 ->
+  // 534 us; 16-token chunks would leave half the waves idle (168 -> 220 us).
+  // At head_dim 256 a workgroup has at least 4 waves: waves past G only
+  // share the loads, and one or two waves would each carry 16-32 loads per
+  // ring stage (register spills). It has at most 8: more than 8 query heads
+  // per KV head go to groups of 8 in workgroups of their own (16 waves cap
+  // the registers at 128, and the head_dim-256 state then spills).
+  const int WG = G <= 1 && g.D < 256 ? 1 : G <= 2 && g.D < 256 ? 2 : G <= 4 ? 4 : G <= 8 || g.D == 256 ? 8 : 16;
+  e.hgroups = (G + WG - 1) / WG;
+  const int TP = (!beside && WG <= 8 && g.D <= 128 && max_q_len > 16) ? 2 : 1;
+  const int W = WG * TP;
+  const int64_t tiles = ((int64_t)max_q_len + 16 * TP - 1) / (16 * TP);
+  // (tile, KV head, head group, sequence) workgroups
+  const int64_t per_split = tiles * g.Hkv * e.hgroups * num_seqs;
+  const void *fn = ext_kernel(g.D, W, TP);
+  // When the launch leaves resident workgroup slots empty (short chunks over
+  // long contexts: one workgroup per (sequence, KV head) streams a whole
+  // context), each key range splits in up to 4, at least 8 steps apiece;
+  // the f32 partials go to the pool-owned workspace and a second launch
+  // merges them. Slots = resident workgroups per CU of this instantiation
+  // (occupancy query, once per pool) x CUs; one per CU beside a decode launch.
+  const int per_cu = ext_resident_per_cu(p, fn, W, TP);
+  const int cus = device_cus(p);
+  const int64_t slots = per_cu > 0 && cus > 0 ? (beside ? 1 : (int64_t)per_cu) * cus : 0;
+  const int64_t steps_max = ((int64_t)(max_ctx_len + kPageSize - 1) / kPageSize + kExtKB - 1) / kExtKB;
+  if (per_split < slots)
+    e.splits = (int32_t)std::min<int64_t>({(int64_t)split_cap, (slots + per_split - 1) / per_split,
+                                           std::max<int64_t>(1, steps_max / 8)});
+  const int64_t rows = (int64_t)num_seqs * max_q_len * g.Hq;  // bounds the (token, query head) rows
+  if (e.splits > 1 || e.partial) {
+    const uint64_t ml_bytes = ((uint64_t)rows * e.splits * 8 + 255) / 256 * 256;
+    const uint64_t need = ml_bytes + (uint64_t)rows * e.splits * g.D * 4;
+    if (p->ws_bytes < need) {
+      const uint64_t cap = std::max<uint64_t>(need, p->ws_bytes + p->ws_bytes / 2);
+      MKV_CHECK_HIP(hipStreamSynchronize(hs));  // earlier launches may read the old buffer
+      if (p->ws) MKV_CHECK_HIP(hipFree(p->ws));
+      p->ws = nullptr;
+      p->ws_bytes = 0;
+      MKV_CHECK_HIP(hipMalloc(&p->ws, cap));
+      p->ws_bytes = cap;
+    }
+    a.ws_ml = reinterpret_cast<float *>(p->ws);
+    a.ws_o = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(p->ws) + ml_bytes);
+  }
+  const int64_t total = per_split * e.splits;  // linear index -> (tile, KV head, group, sequence, split), by XCD
+  e.tiles = (int32_t)tiles;
+  e.per_xcd = (int32_t)((total + 7) / 8);
+  const dim3 grid((unsigned)(8 * (int64_t)e.per_xcd)), block(64 * W);
+  void *args[] = {&a, &e};
+  MKV_CHECK_HIP(hipLaunchKernel(fn, grid, block, args, 0, hs));
+  MKV_CHECK_LAUNCH("attn_extend_kernel");
+  if (e.splits > 1 && !e.partial) {
+    const dim3 mgrid((unsigned)((rows + 3) / 4));
+    switch (g.D) {
+      case 64: hipLaunchKernelGGL((merge_ext_kernel<64, true>), mgrid, dim3(256), 0, hs, a, e); break;
+      case 128: hipLaunchKernelGGL((merge_ext_kernel<128, true>), mgrid, dim3(256), 0, hs, a, e); break;
+      default: hipLaunchKernelGGL((merge_ext_kernel<256, true>), mgrid, dim3(256), 0, hs, a, e); break;
+    }
+    MKV_CHECK_LAUNCH("merge_ext_kernel");
+  }
+  return MKV_OK;
+}
