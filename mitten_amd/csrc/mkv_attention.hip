@@ -608,8 +608,8 @@ __global__ void __launch_bounds__(256) attn_split_kernel(KArgs a, SplitArgs sp) 
 }
 
 // Extend attention on the decode kernels' per-sequence segments, for pools
-// the MFMA extend kernel does not take (f32, head_dim 32, more than 16
-// query heads per KV head): query token t of sequence b, at position p,
+// the extend kernels do not take (head_dim 32, more than 16 query heads per
+// KV head in bf16, or the MKV_ATTN_FORCE_VALU flag): query token t of sequence b, at position p,
 // is decode attention over keys 0..p through b's block table, with q and o
 // rows addressed by t (a virtual sequence per token). One unit per
 // (token, KV head, query-head chunk), whole context, final stores.

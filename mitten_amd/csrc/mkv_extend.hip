@@ -439,6 +439,249 @@ __global__ void __launch_bounds__(64 * W) attn_extend_kernel(KArgs a, ExtArgs e)
                                                           pack_bf16x2(st.O[nn][2] * f, st.O[nn][3] * f));
 }
 
+// ===========================================================================
+// Extend attention of f32 pools (head_dim 64, 128, 256; any group size).
+//
+// The rows of one (sequence, KV head) are its (position, query head of the
+// group) pairs in memory order, row r = position r / G, head r % G, so a tile
+// of rows is full whatever G is. One workgroup per tile of RS * 16 rows; its
+// kExtF32Waves waves take the tile's key blocks in turn (wave w: blocks w,
+// w + kExtF32Waves, ...), each with its own online softmax state, and merge
+// through LDS at the end. A key range cut over the waves keeps the longest
+// serial chain short: these prompts are small, and the last tile of a
+// 512-token prompt bounds the launch. The waves read disjoint blocks, so K and
+// V go from memory straight into the operand layout with no LDS and no barrier
+// in the loop; at head_dim 64 the next block's loads are issued before
+// this one is used.
+//
+// What bounds it: short prompts (8 of 32-512 tokens, 14 query heads, 36.7 us a
+// layer) by the serial chain of a tile, 30% of the f32 matrix rate; long ones
+// by the matrix cores and the softmax between them (8 x 512: 51 TFLOP/s, 64 x
+// 512 after 2,000: 108 of 157). One decode segment per query token, which
+// every f32 prompt took before, read the context once per token: 139 us for
+// the same short prompts. Eight waves per tile: 48.8 us; one 16-row group per
+// workgroup: 37.1 us, and 58 for 102 TFLOP/s at 64 x 512 after 2,000.
+//
+// All in f32 on v_mfma_f32_16x16x4 (twice the rate of unpacked f32 FMAs, and
+// no cross-lane score sums). Lane = (g = lane / 16, c = lane % 16):
+//   S^T = K.Q^T   contraction step 4j + e takes dim 16j + 4g + e from k-slot g:
+//                 one 16-byte load per lane and 16 dims, of K and of Q;
+//   O^T = V^T.P^T step i takes key 4g + i from k-slot g, which is where S^T
+//                 left it; row m of output tile (hh, n) is dim 64hh + 4m + n,
+//                 so one 16-byte load of V row 4g + i feeds four tiles and a
+//                 lane's results are four whole 16-byte chunks per 64 dims.
+// ===========================================================================
+
+constexpr int kExtF32Waves = 4;
+
+template <int D, int RS>
+__global__ void __launch_bounds__(64 * kExtF32Waves) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1)))
+attn_ext_f32_kernel(KArgs a, ExtArgs e) {
+  constexpr int NW = kExtF32Waves, ROWS = 16 * RS;
+  constexpr int NK = D / 16;  // 16-byte chunks of a K or Q row per lane
+  constexpr int NH = D / 64;  // 64-dim runs of a V row: one 16-byte chunk per lane each
+  constexpr int CPR = D / 4;  // 16-byte chunks of a row
+  constexpr int RING = D <= 64 ? 2 : 1;  // blocks in registers (past head_dim 64 a second one spills)
+  __shared__ __attribute__((aligned(16))) float part[NW][ROWS][D];  // unnormalised rows, chunk c at c ^ (row % 16)
+  __shared__ float2 part_ml[NW][ROWS];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g4 = lane >> 4, c16 = lane & 15;
+  // Workgroup -> (tile, KV head, sequence): the tiles with the most keys first,
+  // every (sequence, KV head) in turn, rotated by one per tile. Consecutive
+  // workgroups go to the XCDs in turn, so each sequence's tiles spread over
+  // all of them (a prompt's work grows with the square of its length: one
+  // sequence per XCD, as the bf16 kernel deals them, took 57 us for 37).
+  const int pairs = a.Hkv * e.B, tr = (int)blockIdx.x / pairs;
+  const int pair = ((int)blockIdx.x - tr * pairs + tr) % pairs;
+  const int t = e.tiles - 1 - tr, h = pair % a.Hkv, b = pair / a.Hkv;
+  const int q0 = e.q_indptr[b], nq = e.q_indptr[b + 1] - q0;
+  if (nq == 0) return;
+  const int ctx = e.ctx[b];
+  if (nq < 0 || nq > ctx || ctx > e.max_ctx || q0 < 0 || (int64_t)q0 + nq > (int64_t)e.B * e.max_q) {
+    if (threadIdx.x == 0 && t == 0) record_error(a.d_err, MKV_DEVERR_CTX);
+    return;
+  }
+  const int tab0 = a.indptr[b];
+  if (tab0 < 0 || a.indptr[b + 1] - tab0 < (ctx + kPageSize - 1) / kPageSize) {
+    if (threadIdx.x == 0 && t == 0) record_error(a.d_err, MKV_DEVERR_TABLE);
+    return;
+  }
+  typedef const __attribute__((address_space(4))) int32_t const_i32;
+  const const_i32 *table = (const const_i32 *)(a.ids + tab0);
+  const int rows = nq * a.G;
+  // Lane offsets of its K and V chunks inside a block.
+  const int64_t k_lane = (int64_t)c16 * a.row_bytes + (int64_t)h * D * 4 + 16 * g4;
+  const int64_t v_lane = (int64_t)(4 * g4) * a.row_bytes + (int64_t)h * D * 4 + 16 * c16;
+  const float inv_sl2 = 1.0f / a.sl2;
+
+  // (One tile per workgroup; a chunk longer than max_q_len takes further rounds.)
+  for (int r0 = ROWS * t; r0 < rows; r0 += ROWS * e.tiles) {
+    const int first = ctx - nq + r0 / a.G;                             // the tile's first query position
+    const int n = (ctx - nq + (min(rows, r0 + ROWS) - 1) / a.G) / kPageSize + 1;  // key blocks it sees
+    int qpos[RS];
+    f32x4 qop[RS][NK];
+#pragma unroll
+    for (int s = 0; s < RS; s++) {
+      const int r = min(r0 + 16 * s + c16, rows - 1), pos = r / a.G;
+      qpos[s] = ctx - nq + pos;
+      const float *qp = static_cast<const float *>(a.q) +
+                        ((int64_t)(q0 + pos) * a.Hq + h * a.G + (r - pos * a.G)) * D + 4 * g4;
+#pragma unroll
+      for (int j = 0; j < NK; j++) qop[s][j] = *reinterpret_cast<const f32x4 *>(qp + 16 * j);
+    }
+    f32x4 O[RS][4 * NH];
+    float m[RS], l[RS], thr[RS];
+#pragma unroll
+    for (int s = 0; s < RS; s++) {
+#pragma unroll
+      for (int i = 0; i < 4 * NH; i++) O[s][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      m[s] = thr[s] = -INFINITY;
+      l[s] = 0.0f;
+    }
+    f32x4 kr[RING][NK], vr[RING][4][NH];
+    bool badr[RING];
+    auto issue = [&](f32x4 (&kd)[NK], f32x4 (&vd)[4][NH], bool &bad, int k) {
+      const int32_t blk = table[min(k, n - 1)];  // past the end: the last block again, unused
+      bad = blk < 0 || blk >= a.nblocks;
+      const int64_t off = (int64_t)(bad ? 0 : blk) * a.block_bytes;
+      const uint8_t *kp = a.k_plane + off + k_lane, *vp = a.v_plane + off + v_lane;
+#pragma unroll
+      for (int j = 0; j < NK; j++) kd[j] = *reinterpret_cast<const f32x4 *>(kp + 64 * j);
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int hh = 0; hh < NH; hh++) vd[i][hh] = *reinterpret_cast<const f32x4 *>(vp + i * a.row_bytes + 256 * hh);
+    };
+    auto step = [&](const f32x4 (&kd)[NK], f32x4 (&vd)[4][NH], bool bad, int k) {
+      const int key = kPageSize * k + 4 * g4;  // the lane's first key
+      const bool full = !bad && kPageSize * k + kPageSize - 1 <= first;
+      float p[RS][4];
+#pragma unroll
+      for (int s = 0; s < RS; s++) {
+        // Chains of 8 products, added pairwise: rounds no more often than the
+        // lane partial sums of the decode kernels do (one chain over 64 dims:
+        // twice the error of a score).
+        f32x4 S = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NK; j += 4) {
+          f32x4 c[2][4];
+#pragma unroll
+          for (int y = 0; y < 4; y++) c[0][y] = c[1][y] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int x = 0; x < 4; x++)
+#pragma unroll
+            for (int y = 0; y < 4; y++)
+              c[x >> 1][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(kd[j + y][x], qop[s][j + y][x], c[x >> 1][y], 0, 0, 0);
+          const f32x4 sum = ((c[0][0] + c[1][0]) + (c[0][1] + c[1][1])) + ((c[0][2] + c[1][2]) + (c[0][3] + c[1][3]));
+          S = j ? S + sum : sum;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) p[s][i] = S[i];
+        float mloc = -INFINITY;
+        if (full) {
+          mloc = fmaxf(fmaxf(p[s][0], p[s][1]), fmaxf(p[s][2], p[s][3]));
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            if (!bad && key + i <= qpos[s]) mloc = fmaxf(mloc, p[s][i]);
+        }
+        // Rescale only when a score passes the running max by the slack.
+        if (__ballot(mloc > thr[s])) {
+          mloc = fmaxf(mloc, __shfl_xor(mloc, 16));
+          mloc = fmaxf(mloc, __shfl_xor(mloc, 32));
+          const float ms = mloc * a.sl2;
+          const float mn = ms > m[s] + kRescaleSlack ? ms : m[s];
+          const float al = m[s] == -INFINITY ? 0.0f : fast_exp2(m[s] - mn);
+          l[s] *= al;
+#pragma unroll
+          for (int i = 0; i < 4 * NH; i++) O[s][i] *= al;
+          m[s] = mn;
+          thr[s] = (mn + kRescaleSlack) * inv_sl2;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) p[s][i] = fast_exp2(fmaf(p[s][i], a.sl2, -m[s]));
+        if (!full) {
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            if (bad || key + i > qpos[s]) p[s][i] = 0.0f;
+        }
+        l[s] += (p[s][0] + p[s][1]) + (p[s][2] + p[s][3]);
+      }
+      if (!full) {  // V rows past the context may hold any bit pattern, and 0 * NaN would poison O
+        if (bad && lane == 0) record_error(a.d_err, MKV_DEVERR_BLOCK);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (bad || key + i >= ctx)
+#pragma unroll
+            for (int hh = 0; hh < NH; hh++) vd[i][hh] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int hh = 0; hh < NH; hh++)
+#pragma unroll
+          for (int nn = 0; nn < 4; nn++)
+#pragma unroll
+            for (int s = 0; s < RS; s++)
+              O[s][4 * hh + nn] =
+                  __builtin_amdgcn_mfma_f32_16x16x4f32(vd[i][hh][nn], p[s][i], O[s][4 * hh + nn], 0, 0, 0);
+    };
+    if constexpr (RING == 2) {
+      issue(kr[0], vr[0], badr[0], wave);
+      for (int k = wave; k < n; k += 2 * NW) {
+        issue(kr[1], vr[1], badr[1], k + NW);
+        step(kr[0], vr[0], badr[0], k);
+        issue(kr[0], vr[0], badr[0], k + 2 * NW);
+        if (k + NW < n) step(kr[1], vr[1], badr[1], k + NW);
+      }
+    } else {
+      for (int k = wave; k < n; k += NW) {
+        issue(kr[0], vr[0], badr[0], k);
+        step(kr[0], vr[0], badr[0], k);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < RS; s++) {
+      const int row = 16 * s + c16;
+      l[s] += __shfl_xor(l[s], 16);
+      l[s] += __shfl_xor(l[s], 32);
+      if (g4 == 0) part_ml[wave][row] = make_float2(m[s], l[s]);
+#pragma unroll
+      for (int hh = 0; hh < NH; hh++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          *reinterpret_cast<f32x4 *>(&part[wave][row][((16 * hh + 4 * g4 + i) ^ c16) * 4]) =
+              f32x4{O[s][4 * hh][i], O[s][4 * hh + 1][i], O[s][4 * hh + 2][i], O[s][4 * hh + 3][i]};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int x = 0; x < ROWS * CPR / (64 * NW); x++) {
+      const int at = (int)threadIdx.x + 64 * NW * x;
+      const int row = at / CPR, cc = at % CPR, r = r0 + row;
+      if (r >= rows) break;
+      float M = -INFINITY, L = 0.0f;
+#pragma unroll
+      for (int w = 0; w < NW; w++) M = fmaxf(M, part_ml[w][row].x);
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < NW; w++) {
+        const float2 ml = part_ml[w][row];
+        const float f = ml.x == -INFINITY ? 0.0f : fast_exp2(ml.x - M);
+        L = fmaf(ml.y, f, L);
+        const f32x4 o = *reinterpret_cast<const f32x4 *>(&part[w][row][(cc ^ (row & 15)) * 4]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[i] = fmaf(o[i], f, acc[i]);
+      }
+      const float f = final_scale(M, L, a.zero_sink);
+      const int pos = r / a.G;
+      *reinterpret_cast<f32x4 *>(static_cast<float *>(a.o) +
+                                 ((int64_t)(q0 + pos) * a.Hq + h * a.G + (r - pos * a.G)) * D + 4 * cc) = acc * f;
+    }
+    __syncthreads();  // the next round writes the partials again
+  }
+}
+
 // Log-sum-exp merge of the extend kernel's key-range partials: one wave per
 // (query token, query head) row, partials row * splits + s.
 template <int D, bool BF16>
@@ -454,6 +697,24 @@ __global__ void __launch_bounds__(256) merge_ext_kernel(KArgs a, ExtArgs e) {
 }  // namespace mkv
 
 using namespace mkv;
+
+// The f32 kernel for e (B, max_q, max_ctx and the sequence arguments set).
+static int launch_ext_f32(Pool *p, KArgs &a, ExtArgs &e, hipStream_t hs) {
+  const Geom &g = p->g;
+  const int RS = g.D == 64 ? 2 : 1;  // 16-row groups per workgroup
+  const int64_t tiles = ((int64_t)e.max_q * a.G + 16 * RS - 1) / (16 * RS);
+  const int64_t total = tiles * g.Hkv * e.B;
+  if (tiles > INT32_MAX / 64 || total > INT32_MAX) return set_error(MKV_ERR_INVALID_ARGUMENT, "grid too large");
+  e.tiles = (int32_t)tiles;
+  const dim3 grid((unsigned)total), block(64 * kExtF32Waves);
+  switch (g.D) {
+    case 64: hipLaunchKernelGGL((attn_ext_f32_kernel<64, 2>), grid, block, 0, hs, a, e); break;
+    case 128: hipLaunchKernelGGL((attn_ext_f32_kernel<128, 1>), grid, block, 0, hs, a, e); break;
+    default: hipLaunchKernelGGL((attn_ext_f32_kernel<256, 1>), grid, block, 0, hs, a, e); break;
+  }
+  MKV_CHECK_LAUNCH("attn_ext_f32_kernel");
+  return MKV_OK;
+}
 
 extern "C" int mkv_extend_attention(mkv_pool *pool, int32_t layer, const void *d_q, void *d_o,
                                     const int32_t *d_q_indptr, const int32_t *d_block_indptr,
@@ -477,6 +738,16 @@ extern "C" int mkv_extend_attention(mkv_pool *pool, int32_t layer, const void *d
   if (!aligned16(d_q) || !aligned16(d_o)) return set_error(MKV_ERR_INVALID_ARGUMENT, "q and o must be 16-byte aligned");
   DeviceGuard guard(p->device);
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+  if (g.dtype == MKV_DTYPE_F32 && g.D >= 64 && !(flags & MKV_ATTN_FORCE_VALU)) {
+    KArgs a = make_kargs(p, layer, d_q, d_o, d_block_indptr, d_block_ids, scale, flags, false);
+    ExtArgs e{};
+    e.q_indptr = d_q_indptr;
+    e.ctx = d_ctx_lens;
+    e.B = num_seqs;
+    e.max_ctx = max_ctx_len;
+    e.max_q = max_q_len;
+    return launch_ext_f32(p, a, e, hs);
+  }
   if (!use_mfma || G > 16) {  // per-token segments on the decode kernels
     KArgs a = make_kargs(p, layer, d_q, d_o, d_block_indptr, d_block_ids, scale, flags, use_mfma);
     return launch_ext_segments(p, a, d_q_indptr, d_ctx_lens, num_seqs, max_q_len, max_ctx_len, use_mfma, hs);

@@ -2,9 +2,9 @@
 each sequence's newest tokens attend causally over the whole cache,
 against the oracle (bf16 row-relative 2e-2, f32 max-abs 1e-5), plus the
 identities the oracle tests pin (the chunk's last query equals decode
-attention) and the error paths. Both paths: MFMA query tiles (bf16,
-head_dim 64/128/256, up to 16 query heads per KV head) and per-token
-decode segments (everything else)."""
+attention) and the error paths. Three paths: bf16 MFMA query tiles (head_dim
+64/128/256, up to 16 query heads per KV head), f32 MFMA row tiles (head_dim
+64/128/256) and per-token decode segments (everything else)."""
 from __future__ import annotations
 
 import numpy as np
@@ -29,7 +29,7 @@ SHAPES = {
     "d256-g4": (16, 4, 256),   # head_dim 256 with 4 waves per workgroup
     "d256-g16": (16, 1, 256),  # head_dim 256 with 16 waves per workgroup
 }
-# Shapes the MFMA tile kernel does not take (per-token segments instead).
+# Shapes the bf16 tile kernel does not take (f32 row tiles or per-token segments).
 SEGMENT_SHAPES = {
     # name: (Hq, Hkv, D, dtype)
     "qwen0.5b-f32": (14, 2, 64, "f32"),   # the reference's CPU-runnable configuration
@@ -179,8 +179,8 @@ def test_extend_split_rejects_chunk_past_max_q_len():
 
 @pytest.mark.parametrize("name", list(SEGMENT_SHAPES))
 def test_extend_segment_path_matches_oracle(name):
-    """f32 pools, head_dim 32 and groups above 16 run one decode segment per
-    query token: f32 within max-abs 1e-5, bf16 within row-relative 2e-2."""
+    """f32 pools, head_dim 32 and groups above 16: f32 within max-abs 1e-5,
+    bf16 within row-relative 2e-2."""
     Hq, Hkv, D, dt = SEGMENT_SHAPES[name]
     ctx, nq = [1, 17, 40, 300, 97], [1, 17, 25, 64, 1]
     got, ref, dec, q_indptr = _case((Hq, Hkv, D), ctx, nq, 95, dtype=dt)
@@ -188,3 +188,35 @@ def test_extend_segment_path_matches_oracle(name):
     assert_attention_close(dec, ref[q_indptr[1:] - 1], dt)
     got, ref, _, _ = _case((Hq, Hkv, D), [50, 33], [20, 33], 96, zero_sink=True, dtype=dt)
     assert_attention_close(got, ref, dt)
+
+
+@pytest.mark.parametrize("shape", [(14, 2, 64), (3, 1, 64), (40, 1, 64), (2, 2, 128), (5, 1, 256)])
+def test_extend_f32_row_tiles(shape):
+    """f32 row tiles at their edges: groups that do and do not divide a tile,
+    a single row, contexts ending at, before and after a block's last slot,
+    chunks after a prefix, and stale slots past the context holding NaN."""
+    Hq, Hkv, D = shape
+    ctx, nq = [1, 16, 17, 80, 129, 47, 300], [1, 16, 2, 5, 129, 33, 64]
+    batch = wl.decode_batch_from_contexts([c - 1 for c in ctx], wl.SplitMix64(101), extra_blocks=2)
+    desc = PoolDesc(1, Hkv, Hq, D, batch.num_blocks, "f32")
+    host = normal(102, desc.shape, "f32")
+    stale = host.copy()
+    for b, c in enumerate(ctx):
+        if c % 16:
+            stale[:, :, batch.block_ids[batch.block_indptr[b] + c // 16], c % 16:] = np.nan
+    q_indptr = np.concatenate([[0], np.cumsum(nq)]).astype(np.int32)
+    q = normal(103, (int(q_indptr[-1]), Hq, D), "f32")
+    args = (to_device(q), _i32(q_indptr), _i32(batch.block_indptr), _i32(batch.block_ids), _i32(batch.ctx_lens))
+    with DeviceKvPool(desc) as pool:
+        pool.write(stale)
+        got = to_host(pool.extend_attention(0, *args, max(nq), max(ctx)))
+        pool.check()
+        # a rejected block id: its keys are skipped and the call reports it
+        bad = batch.block_ids.copy()
+        bad[batch.block_indptr[6]] = desc.num_blocks
+        pool.extend_attention(0, args[0], args[1], args[2], _i32(bad), args[4], max(nq), max(ctx))
+        with pytest.raises(DeviceIndexError) as ei:
+            pool.check()
+        assert ei.value.bits & dp.DEVERR_BLOCK
+    ref = orc.extend_attention(odesc(desc), host, 0, q, q_indptr, batch.block_indptr, batch.block_ids, batch.ctx_lens)
+    assert_attention_close(got, ref, "f32")

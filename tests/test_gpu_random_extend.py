@@ -1,5 +1,5 @@
 """Seeded random extend (chunked-prefill) attention: random head shapes (the
-MFMA query tiles and the per-token segment path), batch sizes, cached
+MFMA query tiles, the f32 row tiles and the per-token segment path), batch sizes, cached
 prefixes, chunk lengths (single tokens, whole prompts, chunks after a prefix,
 and sequences with no new token), the zero sink, and the device or host
 metadata form. Each case checks the causal attention of every new token over
