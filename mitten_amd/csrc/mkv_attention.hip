@@ -36,6 +36,7 @@
 #include <new>
 
 #include "mkv_attn.h"
+#include "mkv_plan.h"
 
 namespace mkv {
 
@@ -43,10 +44,6 @@ constexpr int kQChunkMfma = 16;
 constexpr int kQChunkValu = 8;       // query heads per wave on the per-head (VALU) kernels
 constexpr int kQChunkValuSmall = 1;  // the same for launches too small to fill the device (see the plan)
 constexpr int kRing = 3;       // MFMA loop: blocks loaded ahead + 1
-constexpr int kBlockWeight = 8;    // plan: weight of one block in a piece ...
-constexpr int kSwitchWeight = 12;  // ... and of a sequence start inside it (about 1.5 blocks)
-constexpr int kFirstRoundWeight = 116;  // plan: cap of the first-dispatched pieces, percent
-constexpr int kOddXcdWeight = 96;       // plan: cap of pieces dealt to odd-numbered XCDs, percent
 constexpr int kMinPieceBlocks = 4;      // plan: fewest blocks per piece of a small cooperative plan ...
 constexpr int kSmallPlanBlocks = 8;     // ... one with fewer blocks than this per resident workgroup
 constexpr int kCoopRing = 3;   // register stages of the cooperative kernel (one less when
@@ -1741,7 +1738,10 @@ extern "C" int mkv_decode_plan_create(mkv_pool *pool, mkv_decode_plan **out_plan
   pl->pool = reinterpret_cast<Pool *>(pool);
   pl->device = pl->pool->device;
   DeviceGuard guard(pl->device);
-  hipError_t e = hipEventCreateWithFlags(&pl->uploaded, hipEventDisableTiming);
+  // The event only tells the host that the upload has read the pinned buffer,
+  // so it skips the system-scope fence (which would hold the step's first
+  // launch back).
+  hipError_t e = hipEventCreateWithFlags(&pl->uploaded, hipEventDisableTiming | hipEventDisableSystemFence);
   if (e != hipSuccess) {
     delete pl;
     return hip_fail(e, "hipEventCreate");
@@ -1906,10 +1906,9 @@ static int plan_build(mkv_decode_plan *plan, const int32_t *h_ctx_lens, int32_t 
     blk0v[num_seqs] = (int32_t)acc;
   }
   // Piece boundaries: a greedy fill of the flattened blocks under a weight
-  // cap, the smallest that gives at most P pieces. A block weighs
-  // kBlockWeight; a sequence that starts inside a piece (not at its first
-  // block) adds kSwitchWeight, what its predecessor's partial stores and the
-  // Q reload cost that piece (measured: about 1.5 blocks' time).
+  // cap (cut_pieces), the smallest that gives at most P pieces. A sequence
+  // that starts inside a piece adds what its predecessor's partial stores and
+  // the Q reload cost that piece (measured: about 1.5 blocks' time).
   std::vector<int32_t> f0s;
   // With two resident workgroups per CU, the pieces dispatched first (the
   // first `first` indices, one per CU) get kFirstRoundWeight percent of the
@@ -1925,31 +1924,9 @@ static int plan_build(mkv_decode_plan *plan, const int32_t *h_ctx_lens, int32_t 
   // sequences 72.7 -> 73.4% of peak, Gemma-2B MQA 72.3 -> 73.3%). Launches of several rounds, whose freed slots take
   // the next piece whatever its XCD, keep equal caps.
   const bool odd_light = !pieces && resident > 0 && P == resident;
-  auto cut = [&](int64_t cap) {
-    f0s.clear();
-    int64_t w = 0;
-    int cnt = 0;
-    int32_t b = 0;
-    const int64_t cap_first = cap * kFirstRoundWeight / 100;
-    for (int64_t f = 0; f < total; f++) {
-      while (blk0v[b + 1] <= f) b++;
-      int64_t wi = kBlockWeight + ((f == blk0v[b] && cnt > 0) ? kSwitchWeight : 0);
-      const int64_t idx = (int64_t)f0s.size() - 1;  // the piece being filled
-      const int64_t cq0 = idx < first ? cap_first : cap;
-      const int64_t cq = odd_light && (idx & 1) ? cq0 * kOddXcdWeight / 100 : cq0;
-      if (cnt > 0 && (cnt == 64 || w + wi > cq)) {
-        cnt = 0;
-        w = 0;
-        wi = kBlockWeight;
-      }
-      if (cnt == 0) f0s.push_back((int32_t)f);
-      w += wi;
-      cnt++;
-    }
-    f0s.push_back((int32_t)total);
-  };
+  auto cut = [&](int64_t cap) { cut_pieces(blk0v.data(), num_seqs, cap, first, odd_light, f0s); };
   {  // smallest cap giving at most P pieces (the count falls as the cap grows)
-    int64_t lo = kBlockWeight, hi = 64 * (kBlockWeight + kSwitchWeight);
+    int64_t lo = kBlockWeight, hi = kPieceBlocks * (kBlockWeight + kSwitchWeight);
     while (lo < hi) {
       const int64_t mid = (lo + hi) / 2;
       cut(mid);
@@ -2031,11 +2008,9 @@ static int plan_build(mkv_decode_plan *plan, const int32_t *h_ctx_lens, int32_t 
   for (int32_t b = 0; b < num_seqs; b++) {
     const int nb = blk0[b + 1] - blk0[b];
     const int single = snpiece[b] == 1 && !all_partial ? kMetaSingle : 0;
-    for (int j = 0; j < nb; j++) {
-      const int last = j == nb - 1;
-      fseq[blk0[b] + j] = b;
-      fmeta[blk0[b] + j] = (last ? ctx[b] - kPageSize * j : kPageSize) | (last ? kMetaLast : 0) | single;
-    }
+    std::fill_n(fseq + blk0[b], nb, b);
+    std::fill_n(fmeta + blk0[b], nb - 1, kPageSize | single);
+    fmeta[blk0[b] + nb - 1] = (ctx[b] - kPageSize * (nb - 1)) | kMetaLast | single;
   }
   // Block ids in piece order (flattened order: sequence b's first
   // ceil(ctx_b / 16) table entries at seq_blk0[b]), then the prefix ids.
@@ -2044,11 +2019,9 @@ static int plan_build(mkv_decode_plan *plan, const int32_t *h_ctx_lens, int32_t 
   const bool tables = ht.indptr != nullptr;
   if (tables) {
     int32_t *fid = pl->h_meta + flat_off;
-    for (int32_t b = 0; b < num_seqs; b++) {
-      const uint32_t *t = ht.ids + ht.indptr[b];
-      for (int32_t j = 0, nb = blk0[b + 1] - blk0[b]; j < nb; j++) fid[blk0[b] + j] = (int32_t)t[j];
-    }
-    for (int32_t i = 0; i < ht.n_prefix; i++) fid[total + i] = (int32_t)ht.prefix[i];
+    for (int32_t b = 0; b < num_seqs; b++)
+      std::memcpy(fid + blk0[b], ht.ids + ht.indptr[b], (size_t)(blk0[b + 1] - blk0[b]) * 4);
+    if (ht.n_prefix) std::memcpy(fid + total, ht.prefix, (size_t)ht.n_prefix * 4);
   }
   const size_t used = flat_off + (tables ? (size_t)total + ht.n_prefix : 0);
   // A call that brings device tables flattens their ids into a region of its
