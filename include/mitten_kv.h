@@ -398,13 +398,12 @@ MKV_API int mkv_decode_step_shared_prefix(mkv_pool *pool, const mkv_decode_plan 
  * already appended with mkv_append); the query at position p attends keys
  * 0..p. d_q, d_o: [d_q_indptr[num_seqs]][num_q_heads][head_dim].
  * max_q_len / max_ctx_len bound n_b / ctx_b (a larger ctx_b is skipped and
- * reported, MKV_DEVERR_CTX). Any pool: bf16 pools with head_dim 64/128/256
- * and at most 16 query heads per KV head run MFMA query tiles; other pools
- * (head_dim 32, larger bf16 groups) run one decode segment per query token,
- * f32 pools of head_dim 64/128/256 f32 MFMA tiles.
- * When the MFMA tiles would leave the device's resident workgroup slots
- * empty (few short chunks over long contexts), each key range is split in up
- * to 4 and the f32 partials are merged by a second launch; they use the
+ * reported, MKV_DEVERR_CTX). Any pool: pools with head_dim 64/128/256 run
+ * MFMA tiles (bf16 or f32); head_dim 32 runs one decode segment per query
+ * token.
+ * When the bf16 tiles would leave the device's resident workgroup slots
+ * empty (few short chunks over long contexts, at most 16 query heads per KV
+ * head), each key range is split in up to 4 and the f32 partials are merged by a second launch; they use the
  * pool-owned workspace shared with mkv_decode_attention (grown on demand:
  * that call synchronises the stream once, and such calls on one pool must
  * not run concurrently on different streams).

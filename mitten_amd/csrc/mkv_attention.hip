@@ -605,8 +605,7 @@ __global__ void __launch_bounds__(256) attn_split_kernel(KArgs a, SplitArgs sp) 
 }
 
 // Extend attention on the decode kernels' per-sequence segments, for pools
-// the extend kernels do not take (head_dim 32, more than 16 query heads per
-// KV head in bf16, or the MKV_ATTN_FORCE_VALU flag): query token t of sequence b, at position p,
+// the extend kernels do not take (head_dim 32, or the MKV_ATTN_FORCE_VALU flag): query token t of sequence b, at position p,
 // is decode attention over keys 0..p through b's block table, with q and o
 // rows addressed by t (a virtual sequence per token). One unit per
 // (token, KV head, query-head chunk), whole context, final stores.
@@ -617,7 +616,7 @@ struct ExtSplitArgs {
   int32_t B, max_ctx;
 };
 
-template <int D, bool BF16, bool MFMA>
+template <int D, bool BF16, bool MFMA, int QC>
 __global__ void __launch_bounds__(256) attn_ext_split_kernel(KArgs a, ExtSplitArgs x) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -654,7 +653,7 @@ __global__ void __launch_bounds__(256) attn_ext_split_kernel(KArgs a, ExtSplitAr
   sg.j0 = 0;
   sg.j1 = (sg.ctx + kPageSize - 1) / kPageSize;
   sg.nk = sg.nv = nullptr;
-  run_segment<D, BF16, MFMA>(a, sg, lane, true, 0, 1);
+  run_segment<D, BF16, MFMA, QC>(a, sg, lane, true, 0, 1);
 }
 
 template <int D, bool BF16>
@@ -1483,7 +1482,7 @@ KArgs make_kargs(Pool *p, int32_t layer, const void *d_q, void *d_o, const int32
   } while (0)
 
 int launch_ext_segments(Pool *p, KArgs &a, const int32_t *d_q_indptr, const int32_t *d_ctx_lens, int32_t num_seqs,
-                        int32_t max_q_len, int32_t max_ctx_len, bool use_mfma, hipStream_t hs) {
+                        int32_t max_q_len, int32_t max_ctx_len, hipStream_t hs) {
   const Geom &g = p->g;
   const int64_t tokens = (int64_t)num_seqs * max_q_len;  // upper bound; the kernel reads q_indptr[B]
   ExtSplitArgs x;
@@ -1494,7 +1493,7 @@ int launch_ext_segments(Pool *p, KArgs &a, const int32_t *d_q_indptr, const int3
   x.total_units = tokens * g.Hkv * a.nqc;
   const int64_t wgs = (x.total_units + 3) / 4;
   if (wgs > INT32_MAX) return set_error(MKV_ERR_INVALID_ARGUMENT, "launch too large");
-  MKV_DISPATCH(attn_ext_split_kernel, dim3((unsigned)wgs), dim3(256), hs, a, x);
+  MKV_DISPATCH_VALU_QC(attn_ext_split_kernel, kQChunkValu, dim3((unsigned)wgs), dim3(256), hs, a, x);
   MKV_CHECK_LAUNCH("attn_ext_split_kernel");
   return MKV_OK;
 }
@@ -1821,7 +1820,7 @@ static int64_t coop_resident(Pool *p) {
 // pieces, on a second stream. The suffixes are HBM-bound and the prefix is
 // bound by issue and the matrix cores, so a CU that holds one workgroup of
 // each keeps both busy. That pairing fits when the decode kernel and the
-// one-sub-tile prefix instantiation each hold two workgroups per CU: each
+// 8-wave prefix instantiation each hold two workgroups per CU: each
 // then takes at most half of every CU resource. The plan then cuts one
 // suffix piece per CU, and the prefix is split to about one workgroup per
 // CU (Qwen2.5-7B heads, 256 sequences over a 4,100-token prefix: 2.86 ->
@@ -1833,8 +1832,7 @@ static bool prefix_beside(Pool *p) {
     const int G = g.Hq / g.Hkv;
     const int cus = device_cus(p);
     if (cus > 0 && g.D <= 128 && G <= 8 && coop_resident(p) == 2 * (int64_t)cus) {
-      const int WG = G <= 1 ? 1 : G <= 2 ? 2 : G <= 4 ? 4 : 8;
-      if (ext_resident_per_cu(p, ext_kernel(g.D, WG, 1), WG, 1) >= 2) p->beside = 1;
+      if (ext_resident_per_cu(p, ext_kernel(g.D, 8), 8) >= 2) p->beside = 1;
     }
   }
   return p->beside > 0;

@@ -179,13 +179,14 @@ struct ExtArgs {
                             // v_nq queries over v_ctx tokens of the table a.ids (no indptr, no ctx)
   const int32_t *ctx;       // [B] tokens in the cache, the chunk included
   int32_t B, max_ctx;
-  int32_t tiles, per_xcd;   // query tiles per sequence; logical workgroups per XCD
+  int32_t tiles, per_xcd;   // row tiles per (sequence, KV head); logical workgroups per XCD
+  int32_t row_waves;        // waves of a workgroup that hold rows: tiles of 16 * row_waves rows
+  int32_t spread;           // 1: workgroups dealt tile by tile over all sequences (ext_tile)
   int32_t splits;           // key-range splits per (tile, KV head, sequence); > 1: f32 partials + merge
   int32_t max_q;            // max_q_len: with splits, partial rows exist for B * max_q tokens
   int32_t causal;           // 0: every query sees all ctx keys (a shared prefix's decode queries)
   int32_t partial;          // 1: f32 partials whatever the split count, merged by the caller
   int32_t v_nq, v_ctx;      // the one sequence when q_indptr is null
-  int32_t hgroups;          // workgroups per (tile, KV head): each takes W / TP consecutive query heads
 };
 
 // ---- host side ------------------------------------------------------------------
@@ -198,13 +199,12 @@ KArgs make_kargs(Pool *p, int32_t layer, const void *d_q, void *d_o, const int32
 int device_cus(Pool *p);
 // Extend attention by one decode segment per query token (mkv_attention.hip).
 int launch_ext_segments(Pool *p, KArgs &a, const int32_t *d_q_indptr, const int32_t *d_ctx_lens, int32_t num_seqs,
-                        int32_t max_q_len, int32_t max_ctx_len, bool use_mfma, hipStream_t hs);
+                        int32_t max_q_len, int32_t max_ctx_len, hipStream_t hs);
 
-// The extend kernel's instantiation for head_dim D, W waves and TP
-// sub-tiles of 16 positions per workgroup, and its resident workgroups per
-// CU (mkv_extend.hip).
-const void *ext_kernel(int D, int W, int TP);
-int ext_resident_per_cu(Pool *p, const void *fn, int W, int TP);
+// The extend kernel's instantiation for head_dim D and W waves per workgroup,
+// and its resident workgroups per CU (mkv_extend.hip).
+const void *ext_kernel(int D, int W);
+int ext_resident_per_cu(Pool *p, const void *fn, int W);
 int launch_ext_tiles(Pool *p, KArgs &a, ExtArgs &e, int split_cap, hipStream_t hs, bool beside = false);
 
 }  // namespace mkv

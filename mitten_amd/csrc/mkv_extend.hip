@@ -24,16 +24,21 @@ __device__ __forceinline__ int ext_v_swz(int row, int cpr) {
 // with the causal mask of model.rs:542-555 (a key at position j is visible to
 // the query at position p iff j <= p).
 //
-// One workgroup per (query tile of 16 or 32 positions, KV head, sequence,
-// key-range split); per 16-position sub-tile, W/TP >= G waves, wave g
-// computing query head h*G + g for the sub-tile's positions (the MFMA column
-// dimension). The workgroup streams the head's K/V blocks 0..(last tile
+// The rows of one (sequence, KV head) are its (position, query head of the
+// group) pairs in memory order: row r is position r / G, query head h * G +
+// r % G. One workgroup of W waves per (tile of up to 16 W rows, KV head,
+// sequence, key-range split), 16 rows per wave (the MFMA column dimension), so every
+// wave is full whatever G is and a short chunk computes only the waves its
+// rows need (waves per query head, as before, left one of eight idle at G = 7
+// and all of an unused 16-position sub-tile's at work: 281 -> 274 us a layer
+// at 8 x 512 after 4k, 78 -> 62 at 16 chunks of 5-24 tokens after 4-8k). The
+// workgroup streams the head's K/V blocks 0..(last tile
 // position)/16 (its split's share of them) through a double-buffered LDS
 // tile (rows of one head: D*2 bytes; K and V tiles each with their own
 // bank-conflict-free swizzle), loaded cooperatively one step of two blocks
 // ahead; scores, online softmax and the V^T transpose reads follow the
 // decode kernel, with the causal mask applied on blocks that reach past a
-// sub-tile's first position. Steps whose keys every query of the workgroup
+// wave's first position. Steps whose keys every query of the workgroup
 // sees (all but the last one or two of a tile) run a lean form: block ids
 // staged in LDS and checked once, wave-uniform load bases, no masks, and the
 // PV product on one full-rate 16x16x32 MFMA per 16 dims over both blocks.
@@ -54,27 +59,44 @@ constexpr int kExtIdCap = 1024;
 // (L % 8) * per_xcd + L / 8, so each XCD receives a contiguous run of
 // logical indices: the query tiles of one (sequence, KV head) share that
 // XCD's L2 while they stream the same K/V. Logical index = (tiles - 1 -
-// tile) + tiles * (group + hgroups * (head + Hkv * (sequence + B * split)));
-// false for the padding past the last one. `h` returns head * hgroups +
-// group. The last tile of a chunk attends the most keys,
+// tile) + tiles * (head + Hkv * (sequence + B * split)); false for the
+// padding past the last one. The last tile of a chunk attends the most keys,
 // so a sequence's tiles start longest first (causal 2k-token prompts: 518 ->
 // 487 us), leaving the short ones for the tail.
 __device__ __forceinline__ bool ext_tile(const ExtArgs &e, int Hkv, int &t, int &h, int &b, int &sp) {
   const int L = blockIdx.x;
+  if (e.spread) {
+    // Whole prompts, unsplit: tiles longest first over all sequences, every
+    // (KV head, sequence) pair in turn. Where the pairs are a multiple of the
+    // XCDs, rotated by four per tile, so that two XCDs share a pair's tiles
+    // and the XCD of a batch's longest prompt does not finish last, as with
+    // contiguous runs (8 prompts of 300-1,500 tokens 162 -> 100 us a layer);
+    // rotated through all eight, equal prompts lose the L2 (8 x 2,048 tokens
+    // 320 -> 346 us, 8 x 1,500 on one KV head 127 -> 135).
+    const int pairs = Hkv * e.B, tr = L / pairs;
+    if (tr >= e.tiles) return false;
+    const int pair = (int)(((int64_t)L - (int64_t)tr * pairs + (pairs % 8 == 0 ? 4 * (int64_t)tr : 0)) % pairs);
+    sp = 0;
+    t = e.tiles - 1 - tr;
+    h = pair % Hkv;
+    b = pair / Hkv;
+    return true;
+  }
   const int logical = (L & 7) * e.per_xcd + (L >> 3);
-  const int heads = Hkv * e.hgroups;
-  const int per_split = e.tiles * heads * e.B;
+  const int per_split = e.tiles * Hkv * e.B;
   if (logical >= per_split * e.splits) return false;
   const int r = logical % per_split;
   sp = logical / per_split;
   t = e.tiles - 1 - r % e.tiles;
-  h = (r / e.tiles) % heads;
-  b = r / (e.tiles * heads);
+  h = (r / e.tiles) % Hkv;
+  b = r / (e.tiles * Hkv);
   return true;
 }
 
-template <int D, int W, int KB, int R, int TP>
-__global__ void __launch_bounds__(64 * W) attn_extend_kernel(KArgs a, ExtArgs e) {
+template <int D, int W, int KB, int R>
+// (Eight waves at head_dim <= 128: two workgroups per CU, 128 registers.)
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 128 ? (W == 4 ? 2 : 4) : W / 4)))
+attn_extend_kernel(KArgs a, ExtArgs e) {
   constexpr int NR = D / 32, NT = D / 16;
   constexpr int RB = D * 2;                           // LDS tile row: one head's K or V row
   constexpr int CPR = RB / 16;                        // 16-byte chunks per tile row
@@ -83,18 +105,17 @@ __global__ void __launch_bounds__(64 * W) attn_extend_kernel(KArgs a, ExtArgs e)
   constexpr int NCH = KB * BCH;                       // chunks of one step (KB blocks)
   constexpr int LPL = (NCH + 64 * W - 1) / (64 * W);  // loads per lane per step
   static_assert(R % 2 == 0, "even ring: stage s of an unrolled round uses LDS buffer s & 1");
-  constexpr int WG = W / TP;                          // waves per 16-position sub-tile
-  static_assert(W % TP == 0, "whole sub-tiles per workgroup");
   __shared__ __attribute__((aligned(16))) uint8_t tiles[2][KB][2][TILE];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int m16 = lane & 15, g4 = lane >> 4, a4 = m16 >> 2, rq = m16 & 3;
-  int t, hx, b, sp;
-  if (!ext_tile(e, a.Hkv, t, hx, b, sp)) return;
-  const int h = hx / e.hgroups, hg = hx % e.hgroups;  // KV head; group of W / TP query heads
+  int t, h, b, sp;
+  if (!ext_tile(e, a.Hkv, t, h, b, sp)) return;
   const bool virt = e.q_indptr == nullptr;  // one sequence; the host checked its table length
   const int q0 = virt ? 0 : e.q_indptr[b], nq = virt ? e.v_nq : e.q_indptr[b + 1] - q0;
-  if (nq <= 0 || 16 * TP * t >= nq) return;
+  const int rows = nq * a.G;  // row r: position r / G, query head h * G + r % G
+  const int tile_rows = 16 * e.row_waves;  // rows of a tile
+  if (nq <= 0 || tile_rows * t >= rows) return;
   const int ctx = virt ? e.v_ctx : e.ctx[b];
   // (With partials, a chunk longer than max_q_len or a q_indptr past
   // num_seqs * max_q_len tokens would address partial rows past the workspace.)
@@ -113,31 +134,31 @@ __global__ void __launch_bounds__(64 * W) attn_extend_kernel(KArgs a, ExtArgs e)
   // id needs vmcnt(0) before its readfirstlane).
   typedef const __attribute__((address_space(4))) int32_t const_i32;
   const const_i32 *table = (const const_i32 *)(a.ids + tab0);
-  // The workgroup holds TP sub-tiles of 16 positions; wave = (sub-tile, head slot).
-  const int sub = wave / WG, hw = wave % WG;
-  const int row0 = 16 * (TP * t + sub);                  // first chunk row of this wave's sub-tile
-  // Its first query position; without the causal mask every query stands at
-  // the last position and sees all ctx keys.
-  const int qlo = e.causal ? ctx - nq + row0 : ctx - 1;
-  const int qhi_wg = e.causal ? min(ctx - nq + 16 * TP * (t + 1) - 1, ctx - 1) : ctx - 1;
-  const int n = qhi_wg / kPageSize + 1;                  // blocks the workgroup streams: keys 0..qhi_wg
-  const int nw = min(n, (qlo + 15) / kPageSize + 1);     // blocks this wave's sub-tile sees
+  const int row0 = tile_rows * t + 16 * wave;                  // first row of this wave
+  const bool computes = wave < e.row_waves && row0 < rows;  // (waves past the tile's rows only load)
+  const int r = min(row0 + m16, rows - 1), pos = r / a.G;  // this lane's row
+  const int64_t qrow = (int64_t)(q0 + pos) * a.Hq + h * a.G + (r - pos * a.G);
+  // Query positions: this lane's, the wave's first, and the last of the wave
+  // and of the workgroup. Without the causal mask every query stands at the
+  // last position and sees all ctx keys.
+  const int p0 = ctx - nq;
+  const int qp = e.causal ? p0 + pos : ctx - 1;
+  const int qlo = e.causal ? p0 + min(row0, rows - 1) / a.G : ctx - 1;
+  const int qhi = e.causal ? p0 + min(row0 + 15, rows - 1) / a.G : ctx - 1;
+  const int qhi_wg = e.causal ? p0 + (min(tile_rows * (t + 1), rows) - 1) / a.G : ctx - 1;
+  const int n = qhi_wg / kPageSize + 1;           // blocks the workgroup streams: keys 0..qhi_wg
+  const int nw = min(n, qhi / kPageSize + 1);     // blocks this wave's rows see
   // Steps of KB blocks; with splits, this workgroup takes its share of them
   // (a short context can leave a split none: it stores an empty partial).
   const int nsteps_all = (n + KB - 1) / KB;
   const int sps = (nsteps_all + e.splits - 1) / e.splits;
   const int st0 = min(sp * sps, nsteps_all), st1 = min(st0 + sps, nsteps_all);
-  const int hslot = hg * WG + hw;  // this wave's query head among the KV head's G
-  const bool computes = hslot < a.G;
-  const int hq = h * a.G + min(hslot, a.G - 1);
-  const int qp = e.causal ? qlo + m16 : ctx - 1;  // this lane's query position (rows past nq: unused)
   const int64_t spare = dummy_offset(a);
 
-  // Q^T operand: lane holds Q[row 16t + lane%16][32r + 8*(lane/16) .. +8].
+  // Q^T operand: lane holds Q[row0 + lane%16][32r + 8*(lane/16) .. +8].
   bf16x8 qop[NR];
   {
-    const int row = min(row0 + m16, nq - 1);
-    const uint8_t *qp8 = static_cast<const uint8_t *>(a.q) + ((int64_t)(q0 + row) * a.Hq + hq) * D * 2;
+    const uint8_t *qp8 = static_cast<const uint8_t *>(a.q) + qrow * D * 2;
 #pragma unroll
     for (int r = 0; r < NR; r++)
       qop[r] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(qp8 + 2 * (32 * r + 8 * g4)));
@@ -285,7 +306,7 @@ __global__ void __launch_bounds__(64 * W) attn_extend_kernel(KArgs a, ExtArgs e)
 #pragma unroll
     for (int kb = 0; kb < KB; kb++) {
       const int k = step * KB + kb;
-      if (!FAST && k >= nw) {  // uniform: past this sub-tile's last position (or past n in the last step)
+      if (!FAST && k >= nw) {  // uniform: past this wave's last position (or past n in the last step)
 #pragma unroll
         for (int i = 0; i < 4; i++) sr[kb][i] = -INFINITY;
         masked = true;
@@ -296,14 +317,13 @@ __global__ void __launch_bounds__(64 * W) attn_extend_kernel(KArgs a, ExtArgs e)
 #pragma unroll
       for (int r = 0; r < NR; r++) kq[r] = *reinterpret_cast<const u32x4 *>(tk + k_rd[r]);
       f32x4 S = {0.f, 0.f, 0.f, 0.f};
-      // Where one workgroup fills a CU (two sub-tiles, or head_dim 256 with
-      // 8 or more waves) the score MFMAs issue at raised wave priority, so a
+      // Where one workgroup fills a CU (16 waves, or head_dim 256 with 8) the score MFMAs issue at raised wave priority, so a
       // wave that reaches them overtakes the waves busy with exponentials
       // and the matrix pipe stays fed (8 x 512 after 4k: 455 -> 435-445 us at priority 1, about
       // 1% more at 3; head_dim 256: 259 -> 255 us). The same around the PV
-      // products or the load issue gained nothing, and with one sub-tile at
-      // head_dim <= 128 (two workgroups per CU) it cost 16-token chunks 15%.
-      constexpr bool kPrio = TP == 2 || (D == 256 && W >= 8);
+      // products or the load issue gained nothing, and with two workgroups
+      // per CU it cost 16-token chunks 15%.
+      constexpr bool kPrio = W == 16 || (D == 256 && W >= 8);
       if constexpr (kPrio) __builtin_amdgcn_s_setprio(3);
 #pragma unroll
       for (int r = 0; r < NR; r++)
@@ -401,7 +421,7 @@ __global__ void __launch_bounds__(64 * W) attn_extend_kernel(KArgs a, ExtArgs e)
   // Fast steps: [st0, fast_end), blocks below the workgroup's first query
   // position and below ctx (all keys visible to all its queries), with the
   // steps issued R - 1 ahead inside [kfirst, kend).
-  const int fb = e.causal ? min((ctx - nq + 16 * TP * t + 1) / kPageSize, ctx / kPageSize) : ctx / kPageSize;
+  const int fb = e.causal ? min((p0 + tile_rows * t / a.G + 1) / kPageSize, ctx / kPageSize) : ctx / kPageSize;
   const int fast_end = fast ? max(st0, min(min(st1, fb / KB), kend / KB - (R - 1))) : st0;
   const std::integral_constant<bool, true> kFast;
   const std::integral_constant<bool, false> kGeneric;
@@ -421,10 +441,9 @@ __global__ void __launch_bounds__(64 * W) attn_extend_kernel(KArgs a, ExtArgs e)
   if (!computes) return;
   st.l += __shfl_xor(st.l, 16);
   st.l += __shfl_xor(st.l, 32);
-  const int row = row0 + m16;
-  if (row >= nq) return;
+  if (row0 + m16 >= rows) return;
   if (e.splits > 1 || e.partial) {  // f32 partial (m, l, O) of this key range, merged later
-    const int64_t prow = ((int64_t)(q0 + row) * a.Hq + hq) * e.splits + sp;
+    const int64_t prow = qrow * e.splits + sp;
     float *wo = a.ws_o + prow * D + 4 * g4;
 #pragma unroll
     for (int nn = 0; nn < NT; nn++) *reinterpret_cast<f32x4 *>(wo + 16 * nn) = st.O[nn];
@@ -432,7 +451,7 @@ __global__ void __launch_bounds__(64 * W) attn_extend_kernel(KArgs a, ExtArgs e)
     return;
   }
   const float f = final_scale(st.m, st.l, a.zero_sink);
-  uint16_t *op = reinterpret_cast<uint16_t *>(a.o) + ((int64_t)(q0 + row) * a.Hq + hq) * D + 4 * g4;
+  uint16_t *op = reinterpret_cast<uint16_t *>(a.o) + qrow * D + 4 * g4;
 #pragma unroll
   for (int nn = 0; nn < NT; nn++)
     *reinterpret_cast<uint2 *>(op + 16 * nn) = make_uint2(pack_bf16x2(st.O[nn][0] * f, st.O[nn][1] * f),
@@ -734,7 +753,6 @@ extern "C" int mkv_extend_attention(mkv_pool *pool, int32_t layer, const void *d
   if (num_seqs == 0 || max_q_len == 0) return MKV_OK;
   if (max_q_len > max_ctx_len)
     return set_error(MKV_ERR_INVALID_ARGUMENT, "max_q_len %d > max_ctx_len %d", max_q_len, max_ctx_len);
-  const int G = g.Hq / g.Hkv;
   if (!aligned16(d_q) || !aligned16(d_o)) return set_error(MKV_ERR_INVALID_ARGUMENT, "q and o must be 16-byte aligned");
   DeviceGuard guard(p->device);
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
@@ -748,9 +766,9 @@ extern "C" int mkv_extend_attention(mkv_pool *pool, int32_t layer, const void *d
     e.max_q = max_q_len;
     return launch_ext_f32(p, a, e, hs);
   }
-  if (!use_mfma || G > 16) {  // per-token segments on the decode kernels
-    KArgs a = make_kargs(p, layer, d_q, d_o, d_block_indptr, d_block_ids, scale, flags, use_mfma);
-    return launch_ext_segments(p, a, d_q_indptr, d_ctx_lens, num_seqs, max_q_len, max_ctx_len, use_mfma, hs);
+  if (!use_mfma) {  // per-token segments on the decode kernels
+    KArgs a = make_kargs(p, layer, d_q, d_o, d_block_indptr, d_block_ids, scale, flags, false);
+    return launch_ext_segments(p, a, d_q_indptr, d_ctx_lens, num_seqs, max_q_len, max_ctx_len, hs);
   }
   KArgs a = make_kargs(p, layer, d_q, d_o, d_block_indptr, d_block_ids, scale, flags, true);
   ExtArgs e{};
@@ -760,7 +778,8 @@ extern "C" int mkv_extend_attention(mkv_pool *pool, int32_t layer, const void *d
   e.max_ctx = max_ctx_len;
   e.max_q = max_q_len;
   e.causal = 1;
-  return launch_ext_tiles(p, a, e, 4, hs);
+  // More than 16 query heads per KV head: never split, so the call needs no workspace.
+  return launch_ext_tiles(p, a, e, g.Hq / g.Hkv > 16 ? 1 : 4, hs);
 }
 
 extern "C" int mkv_extend_attention_host(mkv_pool *pool, int32_t layer, const void *d_q, void *d_o,
@@ -809,37 +828,24 @@ extern "C" int mkv_extend_attention_host(mkv_pool *pool, int32_t layer, const vo
   return rc ? rc : rr;
 }
 
-// The extend kernel's instantiation for head_dim D, W waves and TP
-// sub-tiles of 16 positions per workgroup.
-const void *mkv::ext_kernel(int D, int W, int TP) {
-  const void *fn = nullptr;
-#define MKV_EXT_FN(DD, TT)                                                                                  \
-  do {                                                                                                      \
-    switch (W / TT) {                                                                                       \
-      case 1: fn = reinterpret_cast<const void *>(&attn_extend_kernel<DD, 1 * TT, kExtKB, kExtR, TT>); break; \
-      case 2: fn = reinterpret_cast<const void *>(&attn_extend_kernel<DD, 2 * TT, kExtKB, kExtR, TT>); break; \
-      case 4: fn = reinterpret_cast<const void *>(&attn_extend_kernel<DD, 4 * TT, kExtKB, kExtR, TT>); break; \
-      case 8: fn = reinterpret_cast<const void *>(&attn_extend_kernel<DD, 8 * TT, kExtKB, kExtR, TT>); break; \
-      default: fn = reinterpret_cast<const void *>(&attn_extend_kernel<DD, 16, kExtKB, kExtR, 1>); break;     \
-    }                                                                                                       \
-  } while (0)
+// The extend kernel's instantiation for head_dim D and W waves (4, 8 or 16; 4
+// or 8 at head_dim 256: 16 waves cap the registers at 128, and its state then
+// spills).
+const void *mkv::ext_kernel(int D, int W) {
+#define MKV_EXT_FN(DD, WW) reinterpret_cast<const void *>(&attn_extend_kernel<DD, WW, kExtKB, kExtR>)
   switch (D) {
-    case 64: if (TP == 2) MKV_EXT_FN(64, 2); else MKV_EXT_FN(64, 1); break;
-    case 128: if (TP == 2) MKV_EXT_FN(128, 2); else MKV_EXT_FN(128, 1); break;
-    default:
-      fn = W == 4 ? reinterpret_cast<const void *>(&attn_extend_kernel<256, 4, kExtKB, kExtR, 1>)
-                  : reinterpret_cast<const void *>(&attn_extend_kernel<256, 8, kExtKB, kExtR, 1>);
-      break;
+    case 64: return W == 4 ? MKV_EXT_FN(64, 4) : W == 8 ? MKV_EXT_FN(64, 8) : MKV_EXT_FN(64, 16);
+    case 128: return W == 4 ? MKV_EXT_FN(128, 4) : W == 8 ? MKV_EXT_FN(128, 8) : MKV_EXT_FN(128, 16);
+    default: return W == 4 ? MKV_EXT_FN(256, 4) : MKV_EXT_FN(256, 8);
   }
 #undef MKV_EXT_FN
-  return fn;
 }
 
 // Resident workgroups per CU of an extend instantiation (occupancy query,
 // once per pool and instantiation); -1 when unknown.
-int mkv::ext_resident_per_cu(Pool *p, const void *fn, int W, int TP) {
+int mkv::ext_resident_per_cu(Pool *p, const void *fn, int W) {
   const Geom &g = p->g;
-  int &per_cu = p->ext_per_cu[g.D == 64 ? 0 : g.D == 128 ? 1 : 2][W == 1 ? 0 : W == 2 ? 1 : W == 4 ? 2 : W == 8 ? 3 : 4][TP - 1];
+  int &per_cu = p->ext_per_cu[g.D == 64 ? 0 : g.D == 128 ? 1 : 2][W == 4 ? 0 : W == 8 ? 1 : 2];
   if (per_cu == 0) {
     int n_cu = 0;
     DeviceGuard guard(p->device);
@@ -858,7 +864,7 @@ int mkv::ext_resident_per_cu(Pool *p, const void *fn, int W, int TP) {
 // partials are stored, launches, and merges the splits unless e.partial
 // (then a.ws_ml / a.ws_o and e.splits describe the partials left). With
 // beside, the tiles share the device with a decode launch that holds one
-// workgroup per CU: one sub-tile per workgroup, and the split aims at one
+// workgroup per CU: at most 8 waves per workgroup, and the split aims at one
 // workgroup per CU.
 int mkv::launch_ext_tiles(Pool *p, KArgs &a, ExtArgs &e, int split_cap, hipStream_t hs, bool beside) {
   const Geom &g = p->g;
@@ -866,40 +872,59 @@ int mkv::launch_ext_tiles(Pool *p, KArgs &a, ExtArgs &e, int split_cap, hipStrea
   const int64_t num_seqs = e.B, max_q_len = e.max_q, max_ctx_len = e.max_ctx;
   if (((max_q_len + 15) / 16 * g.Hq * num_seqs) * split_cap + 8 > INT32_MAX)
     return set_error(MKV_ERR_INVALID_ARGUMENT, "grid too large");
-  e.splits = 1;
-  // Waves per 16-position sub-tile: the next power of two >= G. Two
-  // sub-tiles per workgroup share each K/V tile (K/V streamed once per 32
-  // positions) where that stays within 16 waves and their register budget
-  // (head_dim <= 128) and chunks are longer than one sub-tile. Measured at
-  // Qwen-7B heads: 8 x 512 after 4k 526 -> 480 us, 8 x 2,048 prompts 560 ->
-  // 534 us; 16-token chunks would leave half the waves idle (168 -> 220 us).
-  // At head_dim 256 a workgroup has at least 4 waves: waves past G only
-  // share the loads, and one or two waves would each carry 16-32 loads per
-  // ring stage (register spills). It has at most 8: more than 8 query heads
-  // per KV head go to groups of 8 in workgroups of their own (16 waves cap
-  // the registers at 128, and the head_dim-256 state then spills).
-  const int WG = G <= 1 && g.D < 256 ? 1 : G <= 2 && g.D < 256 ? 2 : G <= 4 ? 4 : G <= 8 || g.D == 256 ? 8 : 16;
-  e.hgroups = (G + WG - 1) / WG;
-  const int TP = (!beside && WG <= 8 && g.D <= 128 && max_q_len > 16) ? 2 : 1;
-  const int W = WG * TP;
-  const int64_t tiles = ((int64_t)max_q_len + 16 * TP - 1) / (16 * TP);
-  // (tile, KV head, head group, sequence) workgroups
-  const int64_t per_split = tiles * g.Hkv * e.hgroups * num_seqs;
-  const void *fn = ext_kernel(g.D, W, TP);
-  // When the launch leaves resident workgroup slots empty (short chunks over
-  // long contexts: one workgroup per (sequence, KV head) streams a whole
-  // context), each key range splits in up to 4, at least 8 steps apiece;
-  // the f32 partials go to the pool-owned workspace and a second launch
-  // merges them. Slots = resident workgroups per CU of this instantiation
-  // (occupancy query, once per pool) x CUs; one per CU beside a decode launch.
-  const int per_cu = ext_resident_per_cu(p, fn, W, TP);
+  // Waves per workgroup: enough for the longest chunk's rows, at most 16 (8 at
+  // head_dim 256 and beside a decode launch), so that a K/V tile in LDS serves
+  // as many rows as it can; at least 4, since waves past the last row still
+  // share the loads.
+  const int64_t rows_max = max_q_len * G;
+  const int most = beside || g.D == 256 ? 8 : 16;
+  const int W = rows_max <= 64 ? 4 : rows_max <= 128 ? 8 : most;
+  const void *fn = ext_kernel(g.D, W);
+  const int64_t rows = (int64_t)num_seqs * max_q_len * g.Hq;  // bounds the (token, query head) rows
+  // Slots = resident workgroups per CU of this instantiation (occupancy query,
+  // once per pool) x CUs; one per CU beside a decode launch.
+  const int per_cu = ext_resident_per_cu(p, fn, W);
   const int cus = device_cus(p);
   const int64_t slots = per_cu > 0 && cus > 0 ? (beside ? 1 : (int64_t)per_cu) * cus : 0;
   const int64_t steps_max = ((int64_t)(max_ctx_len + kPageSize - 1) / kPageSize + kExtKB - 1) / kExtKB;
-  if (per_split < slots)
-    e.splits = (int32_t)std::min<int64_t>({(int64_t)split_cap, (slots + per_split - 1) / per_split,
-                                           std::max<int64_t>(1, steps_max / 8)});
-  const int64_t rows = (int64_t)num_seqs * max_q_len * g.Hq;  // bounds the (token, query head) rows
+  // Row waves per tile and key-range splits: the pair whose rounds of resident
+  // workgroups take least. A step of a workgroup costs kExtStepWaves + its row
+  // waves (8 x 512 after 4k: two rounds of 16 row waves 317 us, of 14 300 us),
+  // so full tiles are best until a smaller one saves part of a round. A key
+  // range splits where the launch leaves resident slots empty (short chunks
+  // over long contexts: one workgroup per (sequence, KV head) would stream a
+  // whole context), in at most split_cap of at least 8 steps apiece; the f32
+  // partials go to the pool-owned workspace and a second launch merges them
+  // (kExtMergeCost, and each partial's write and read).
+  constexpr double kExtStepWaves = 22, kExtMergeCost = 150, kExtCostPerUs = 36;
+  // Mean keys of a tile over the longest: whole prompts' tiles shrink from
+  // longest to shortest and fill a started round, equal ones do not.
+  const double share = e.causal ? 1.0 - 0.5 * (double)max_q_len / (double)max_ctx_len : 1.0;
+  e.splits = 1;
+  e.row_waves = W;
+  if (slots > 0) {
+    double best = INFINITY;
+    // No split is faster than the K/V bytes (of contexts of 0.6 of the longest).
+    const double kv_cost = kExtCostPerUs * 0.6 * (double)num_seqs * (double)max_ctx_len * 2 * (double)g.row_bytes / 5.5e6;
+    const int64_t most_splits = std::max<int64_t>(1, std::min<int64_t>(split_cap, steps_max / 8));
+    for (int k = W; 2 * k > W; k--) {
+      const int64_t wgs = (rows_max + 16 * k - 1) / (16 * k) * g.Hkv * num_seqs;
+      for (int64_t sp = 1; sp <= (wgs < slots ? most_splits : 1); sp++) {
+        const double x = (double)(wgs * sp) / (double)slots;
+        const double rounds = share > 0.85 ? (x <= 4 ? std::ceil(x) : x + 0.5) : std::max(1.0, x * share + 0.25);
+        double cost = rounds * (double)((steps_max + sp - 1) / sp) * (kExtStepWaves + k);
+        cost = std::max(cost, kv_cost);
+        if (sp > 1) cost += kExtMergeCost + kExtCostPerUs * ((double)rows * sp * g.D * 8 / 5e6);
+        if (cost < best) {
+          best = cost;
+          e.row_waves = k;
+          e.splits = (int32_t)sp;
+        }
+      }
+    }
+  }
+  const int64_t tiles = (rows_max + 16 * e.row_waves - 1) / (16 * e.row_waves);
+  const int64_t per_split = tiles * g.Hkv * num_seqs;  // (tile, KV head, sequence) workgroups
   if (e.splits > 1 || e.partial) {
     const uint64_t ml_bytes = ((uint64_t)rows * e.splits * 8 + 255) / 256 * 256;
     const uint64_t need = ml_bytes + (uint64_t)rows * e.splits * g.D * 4;
@@ -915,9 +940,10 @@ int mkv::launch_ext_tiles(Pool *p, KArgs &a, ExtArgs &e, int split_cap, hipStrea
     a.ws_ml = reinterpret_cast<float *>(p->ws);
     a.ws_o = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(p->ws) + ml_bytes);
   }
-  const int64_t total = per_split * e.splits;  // linear index -> (tile, KV head, group, sequence, split), by XCD
+  const int64_t total = per_split * e.splits;  // linear index -> (tile, KV head, sequence, split), by XCD
   e.tiles = (int32_t)tiles;
   e.per_xcd = (int32_t)((total + 7) / 8);
+  e.spread = share <= 0.85 && e.splits == 1;
   const dim3 grid((unsigned)(8 * (int64_t)e.per_xcd)), block(64 * W);
   void *args[] = {&a, &e};
   MKV_CHECK_HIP(hipLaunchKernel(fn, grid, block, args, 0, hs));

@@ -61,7 +61,7 @@ struct Pool {
   uint64_t ws_bytes = 0;
   int64_t coop_slots = -1;   // resident workgroups of the decode kernel (-1: not yet queried)
   int cus = 0;               // compute units of the device (0: not yet queried)
-  int ext_per_cu[3][5][2] = {};  // resident extend workgroups per CU by (head_dim, waves, sub-tiles); 0: not yet queried
+  int ext_per_cu[3][3] = {};  // resident extend workgroups per CU by (head_dim, waves); 0: not yet queried
   // The shared-prefix step's second stream, which runs the prefix tiles
   // beside the suffix pieces, and its fork / join events (created on first
   // use). beside: 1 when one prefix workgroup fits beside one decode-kernel

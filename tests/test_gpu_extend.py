@@ -2,9 +2,8 @@
 each sequence's newest tokens attend causally over the whole cache,
 against the oracle (bf16 row-relative 2e-2, f32 max-abs 1e-5), plus the
 identities the oracle tests pin (the chunk's last query equals decode
-attention) and the error paths. Three paths: bf16 MFMA query tiles (head_dim
-64/128/256, up to 16 query heads per KV head), f32 MFMA row tiles (head_dim
-64/128/256) and per-token decode segments (everything else)."""
+attention) and the error paths. Three paths: bf16 and f32 MFMA row tiles
+(head_dim 64/128/256) and per-token decode segments (head_dim 32)."""
 from __future__ import annotations
 
 import numpy as np
@@ -29,7 +28,7 @@ SHAPES = {
     "d256-g4": (16, 4, 256),   # head_dim 256 with 4 waves per workgroup
     "d256-g16": (16, 1, 256),  # head_dim 256 with 16 waves per workgroup
 }
-# Shapes the bf16 tile kernel does not take (f32 row tiles or per-token segments).
+# Shapes beside the engine's bf16 ones: f32, head_dim 32, large groups.
 SEGMENT_SHAPES = {
     # name: (Hq, Hkv, D, dtype)
     "qwen0.5b-f32": (14, 2, 64, "f32"),   # the reference's CPU-runnable configuration
@@ -179,8 +178,8 @@ def test_extend_split_rejects_chunk_past_max_q_len():
 
 @pytest.mark.parametrize("name", list(SEGMENT_SHAPES))
 def test_extend_segment_path_matches_oracle(name):
-    """f32 pools, head_dim 32 and groups above 16: f32 within max-abs 1e-5,
-    bf16 within row-relative 2e-2."""
+    """f32 row tiles, a group above 16 on the bf16 tiles, and head_dim 32 on
+    per-token segments: f32 within max-abs 1e-5, bf16 within row-relative 2e-2."""
     Hq, Hkv, D, dt = SEGMENT_SHAPES[name]
     ctx, nq = [1, 17, 40, 300, 97], [1, 17, 25, 64, 1]
     got, ref, dec, q_indptr = _case((Hq, Hkv, D), ctx, nq, 95, dtype=dt)
@@ -220,3 +219,21 @@ def test_extend_f32_row_tiles(shape):
         assert ei.value.bits & dp.DEVERR_BLOCK
     ref = orc.extend_attention(odesc(desc), host, 0, q, q_indptr, batch.block_indptr, batch.block_ids, batch.ctx_lens)
     assert_attention_close(got, ref, "f32")
+
+
+@pytest.mark.parametrize("shape", [(6, 2, 64), (5, 1, 128), (40, 2, 128), (1, 1, 64), (6, 2, 256)])
+@pytest.mark.parametrize("chunks", [
+    # (contexts, new tokens): ragged whole prompts (tiles dealt over all
+    # sequences) with and without a multiple of 8 (KV head, sequence) pairs,
+    # one row, and chunks whose last wave or tile is nearly empty
+    ([1, 16, 17, 80, 129, 47, 300, 333], [1, 16, 17, 80, 129, 47, 300, 333]),
+    ([257, 3, 40], [257, 3, 40]),
+    ([500], [1]),
+    ([700, 90, 400], [52, 4, 13]),
+])
+def test_extend_row_tiles(shape, chunks):
+    """bf16 row tiles (row = position * group + head) for groups that do not
+    divide a wave's 16 rows, at the edges of waves, tiles and workgroups."""
+    ctx, nq = chunks
+    got, ref, _, _ = _case(shape, ctx, nq, 104)
+    assert_attention_close(got, ref, "bf16")

@@ -28,7 +28,7 @@ KINDS = [
     (16, 4, 256, "bf16"),
     (16, 1, 256, "bf16"),
     (14, 2, 64, "f32"),
-    (64, 2, 128, "bf16"),  # 32 query heads per KV head: per-token segments
+    (64, 2, 128, "bf16"),  # 32 query heads per KV head
     (8, 2, 32, "bf16"),    # head_dim 32: per-token segments
 ]
 
