@@ -397,10 +397,14 @@ MKV_API int mkv_decode_step_shared_prefix(mkv_pool *pool, const mkv_decode_plan 
  * positions [ctx_b - n_b, ctx_b) (ctx_b = d_ctx_lens[b], the chunk's K/V
  * already appended with mkv_append); the query at position p attends keys
  * 0..p. d_q, d_o: [d_q_indptr[num_seqs]][num_q_heads][head_dim].
- * max_q_len / max_ctx_len bound n_b / ctx_b (a larger ctx_b is skipped and
- * reported, MKV_DEVERR_CTX). Any pool: pools with head_dim 64/128/256 run
- * MFMA tiles (bf16 or f32); head_dim 32 runs one decode segment per query
- * token.
+ * max_q_len / max_ctx_len bound n_b / ctx_b: a larger ctx_b is skipped and
+ * reported (MKV_DEVERR_CTX), and so is a chunk that starts before row 0; a
+ * larger n_b is computed all the same, but later than its share of the launch.
+ * (Where key ranges are split, see below, a chunk past num_seqs * max_q_len
+ * tokens from d_q_indptr[0] on is skipped and reported; at head_dim 32 tokens
+ * past num_seqs * max_q_len are skipped.) Any pool: pools with head_dim
+ * 64/128/256 run MFMA tiles (bf16 or f32); head_dim 32 runs one decode segment
+ * per query token.
  * When the bf16 tiles would leave the device's resident workgroup slots
  * empty (few short chunks over long contexts, at most 16 query heads per KV
  * head), each key range is split in up to 4 and the f32 partials are merged by a second launch; they use the

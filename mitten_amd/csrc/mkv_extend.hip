@@ -93,10 +93,11 @@ __device__ __forceinline__ bool ext_tile(const ExtArgs &e, int Hkv, int &t, int 
   return true;
 }
 
+// One row tile t of (KV head h, sequence of nq queries from token q0 over ctx
+// keys, its table at a.ids + tab0), key-range split sp.
 template <int D, int W, int KB, int R>
-// (Eight waves at head_dim <= 128: two workgroups per CU, 128 registers.)
-__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 128 ? (W == 4 ? 2 : 4) : W / 4)))
-attn_extend_kernel(KArgs a, ExtArgs e) {
+__device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, int t, int h, int sp, int q0, int nq,
+                                            int ctx, int tab0, int part0) {
   constexpr int NR = D / 32, NT = D / 16;
   constexpr int RB = D * 2;                           // LDS tile row: one head's K or V row
   constexpr int CPR = RB / 16;                        // 16-byte chunks per tile row
@@ -106,29 +107,16 @@ attn_extend_kernel(KArgs a, ExtArgs e) {
   constexpr int LPL = (NCH + 64 * W - 1) / (64 * W);  // loads per lane per step
   static_assert(R % 2 == 0, "even ring: stage s of an unrolled round uses LDS buffer s & 1");
   __shared__ __attribute__((aligned(16))) uint8_t tiles[2][KB][2][TILE];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // (Opaque, as the kernel's arguments: no lane offset is kept in registers
+  // from round to round.)
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  tid &= 64 * W - 1;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m16 = lane & 15, g4 = lane >> 4, a4 = m16 >> 2, rq = m16 & 3;
-  int t, h, b, sp;
-  if (!ext_tile(e, a.Hkv, t, h, b, sp)) return;
-  const bool virt = e.q_indptr == nullptr;  // one sequence; the host checked its table length
-  const int q0 = virt ? 0 : e.q_indptr[b], nq = virt ? e.v_nq : e.q_indptr[b + 1] - q0;
   const int rows = nq * a.G;  // row r: position r / G, query head h * G + r % G
   const int tile_rows = 16 * e.row_waves;  // rows of a tile
-  if (nq <= 0 || tile_rows * t >= rows) return;
-  const int ctx = virt ? e.v_ctx : e.ctx[b];
-  // (With partials, a chunk longer than max_q_len or a q_indptr past
-  // num_seqs * max_q_len tokens would address partial rows past the workspace.)
-  if ((e.causal && nq > ctx) || ctx < 1 || ctx > e.max_ctx ||
-      ((e.splits > 1 || e.partial) && (nq > e.max_q || q0 < 0 || (int64_t)q0 + nq > (int64_t)e.B * e.max_q))) {
-    if (threadIdx.x == 0 && t == 0) record_error(a.d_err, MKV_DEVERR_CTX);
-    return;
-  }
-  const int tab0 = virt ? 0 : a.indptr[b], nbt = (ctx + kPageSize - 1) / kPageSize;
-  if (!virt && (tab0 < 0 || a.indptr[b + 1] - tab0 < nbt)) {
-    if (threadIdx.x == 0 && t == 0) record_error(a.d_err, MKV_DEVERR_TABLE);
-    return;
-  }
   // The table is read through the constant address space: scalar loads,
   // whose wait does not drain the vector-load ring (a vector load of a block
   // id needs vmcnt(0) before its readfirstlane).
@@ -154,6 +142,7 @@ attn_extend_kernel(KArgs a, ExtArgs e) {
   const int sps = (nsteps_all + e.splits - 1) / e.splits;
   const int st0 = min(sp * sps, nsteps_all), st1 = min(st0 + sps, nsteps_all);
   const int64_t spare = dummy_offset(a);
+  const int64_t v_off = a.v_plane - a.k_plane;
 
   // Q^T operand: lane holds Q[row0 + lane%16][32r + 8*(lane/16) .. +8].
   bf16x8 qop[NR];
@@ -184,14 +173,14 @@ attn_extend_kernel(KArgs a, ExtArgs e) {
     }
 #pragma unroll
     for (int i = 0; i < LPL; i++) {
-      const int c = (int)threadIdx.x + 64 * W * i;
+      const int c = tid + 64 * W * i;
       const int kb = min(c / BCH, KB - 1), rem = c % BCH;
       const int kv = rem / (16 * CPR), rem2 = rem % (16 * CPR), row = rem2 / CPR, cc = rem2 % CPR;
       int32_t bk = blk[0];
 #pragma unroll
       for (int j = 1; j < KB; j++) bk = kb == j ? blk[j] : bk;
       const bool real = c < NCH && step * KB + kb < n;
-      const uint8_t *plane = kv ? a.v_plane : a.k_plane;
+      const uint8_t *plane = a.k_plane + (kv ? v_off : 0);
       const int64_t off = real ? (int64_t)bk * a.block_bytes + (int64_t)row * a.row_bytes + h * RB + 16 * cc
                                : spare + 16 * (lane & 7);
       d[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>((real ? plane : a.k_plane) + off));
@@ -213,7 +202,7 @@ attn_extend_kernel(KArgs a, ExtArgs e) {
   if (fast) {
     int badl = 0;
     const int32_t *tg = a.ids + tab0 + kfirst;
-    for (int i = (int)threadIdx.x; i < kend - kfirst; i += 64 * W) {
+    for (int i = tid; i < kend - kfirst; i += 64 * W) {
       const int32_t id = tg[i];
       badl |= (id < 0) | (id >= a.nblocks);
       ids_s[i] = id;
@@ -236,7 +225,7 @@ attn_extend_kernel(KArgs a, ExtArgs e) {
     const int cu = min(cw, NCH - 64);
     const int pl = cu / (16 * CPR), kv = pl & 1;
     fkb[i] = pl >> 1;
-    fpl[i] = kv ? a.v_plane : a.k_plane;
+    fpl[i] = a.k_plane + (kv ? v_off : 0);
     const int rem2 = cu % (16 * CPR) + lane, row = rem2 / CPR, cc = rem2 % CPR;
     flo[i] = (uint32_t)(row * (int)a.row_bytes + h * RB + 16 * cc);
     fwr[i] = (uint32_t)((2 * fkb[i] + kv) * TILE + row * RB + ((cc ^ (kv ? ext_v_swz(row, CPR) : ext_k_swz(row, CPR))) << 4));
@@ -282,7 +271,7 @@ attn_extend_kernel(KArgs a, ExtArgs e) {
         if (kAllVal || fval[i]) *reinterpret_cast<u32x4 *>(&tiles[s & 1][0][0][0] + fwr[i]) = ring[s][i];
         continue;
       }
-      const int c = (int)threadIdx.x + 64 * W * i;
+      const int c = tid + 64 * W * i;
       if (c < NCH) {
         const int kb = c / BCH, rem = c % BCH;
         const int kv = rem / (16 * CPR), rem2 = rem % (16 * CPR), row = rem2 / CPR, cc = rem2 % CPR;
@@ -426,6 +415,9 @@ attn_extend_kernel(KArgs a, ExtArgs e) {
   const std::integral_constant<bool, true> kFast;
   const std::integral_constant<bool, false> kGeneric;
   int k0 = st0;
+  // (No scalar load left in flight: in the loop the compiler would then wait
+  // for every LDS access where it could wait for the oldest.)
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
   for (int it = 0, nit = (fast_end - st0) / R; it < nit; it++, k0 += R) {
 #pragma unroll
     for (int s = 0; s < R; s++) stage(kFast, s, k0 + s);
@@ -443,7 +435,7 @@ attn_extend_kernel(KArgs a, ExtArgs e) {
   st.l += __shfl_xor(st.l, 32);
   if (row0 + m16 >= rows) return;
   if (e.splits > 1 || e.partial) {  // f32 partial (m, l, O) of this key range, merged later
-    const int64_t prow = qrow * e.splits + sp;
+    const int64_t prow = (qrow - (int64_t)part0 * a.Hq) * e.splits + sp;
     float *wo = a.ws_o + prow * D + 4 * g4;
 #pragma unroll
     for (int nn = 0; nn < NT; nn++) *reinterpret_cast<f32x4 *>(wo + 16 * nn) = st.O[nn];
@@ -456,6 +448,57 @@ attn_extend_kernel(KArgs a, ExtArgs e) {
   for (int nn = 0; nn < NT; nn++)
     *reinterpret_cast<uint2 *>(op + 16 * nn) = make_uint2(pack_bf16x2(st.O[nn][0] * f, st.O[nn][1] * f),
                                                           pack_bf16x2(st.O[nn][2] * f, st.O[nn][3] * f));
+}
+
+template <int D, int W, int KB, int R>
+// (Eight waves at head_dim <= 128: two workgroups per CU, 128 registers. The
+// upper bound keeps the scheduler from saving registers for a fifth wave per
+// SIMD, which serialised the V reads: 31.5 -> 34.6 us for one token after 8k
+// at head_dim 64.)
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 128 ? (W == 4 ? 2 : 4) : W / 4, D <= 128 ? 4 : W / 4)))
+attn_extend_kernel(KArgs, ExtArgs) {
+  // One tile per workgroup; a chunk longer than max_q_len takes further rounds.
+  // Each round reads the arguments again, through a pointer that the compiler
+  // cannot see through: kept from round to round, they and what follows from
+  // them spilled at 16 and 8 waves (12-44 bytes a lane at head_dim 128). The
+  // loop costs head_dim 64 up to 5% (16 chunks of 5-24 tokens 32 -> 33.9 us),
+  // 128 nothing, and 256 gains from the arguments not kept (10%).
+  static_assert(sizeof(KArgs) % alignof(ExtArgs) == 0, "ExtArgs follows KArgs");
+  for (int round = 0;; round++) {
+    typedef const __attribute__((address_space(4))) uint8_t const_u8;
+    const_u8 *ka = (const_u8 *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(ka));
+    const KArgs a = *(const KArgs *)ka;
+    const ExtArgs e = *(const ExtArgs *)(ka + sizeof(KArgs));
+    typedef const __attribute__((address_space(4))) int32_t const_i32;  // scalar loads, as the table's
+    const const_i32 *q_indptr = (const const_i32 *)e.q_indptr, *indptr = (const const_i32 *)a.indptr;
+    const const_i32 *ctx_lens = (const const_i32 *)e.ctx;
+    int t, h, b, sp;
+    if (!ext_tile(e, a.Hkv, t, h, b, sp)) return;
+    const bool virt = e.q_indptr == nullptr;  // one sequence; the host checked its table length
+    const int q0 = virt ? 0 : q_indptr[b], nq = virt ? e.v_nq : q_indptr[b + 1] - q0;
+    const int64_t rows = (int64_t)nq * a.G, tile_rows = 16 * e.row_waves;
+    const int64_t tt = t + (int64_t)e.tiles * round;
+    if (nq <= 0 || tile_rows * tt >= rows) return;
+    const int ctx = virt ? e.v_ctx : ctx_lens[b];
+    // Partial rows exist for num_seqs * max_q_len tokens from q_indptr[0] on.
+    const bool parts = e.splits > 1 || e.partial;
+    const int part0 = parts && !virt ? q_indptr[0] : 0;
+    if ((e.causal && nq > ctx) || ctx < 1 || ctx > e.max_ctx || q0 < 0 ||
+        (parts && (q0 < part0 || (int64_t)q0 - part0 + nq > (int64_t)e.B * e.max_q))) {
+      if (threadIdx.x == 0 && t == 0) record_error(a.d_err, MKV_DEVERR_CTX);
+      return;
+    }
+    const int tab0 = virt ? 0 : indptr[b], nbt = (ctx + kPageSize - 1) / kPageSize;
+    if (!virt && (tab0 < 0 || indptr[b + 1] - tab0 < nbt)) {
+      if (threadIdx.x == 0 && t == 0) record_error(a.d_err, MKV_DEVERR_TABLE);
+      return;
+    }
+    const bool more = tile_rows * (tt + e.tiles) < rows;
+    extend_tile<D, W, KB, R>(a, e, (int)tt, h, sp, q0, nq, ctx, tab0, part0);
+    if (!more) return;
+    __syncthreads();  // the next round writes the LDS tiles and ids again
+  }
 }
 
 // ===========================================================================
@@ -517,7 +560,7 @@ attn_ext_f32_kernel(KArgs a, ExtArgs e) {
   const int q0 = e.q_indptr[b], nq = e.q_indptr[b + 1] - q0;
   if (nq == 0) return;
   const int ctx = e.ctx[b];
-  if (nq < 0 || nq > ctx || ctx > e.max_ctx || q0 < 0 || (int64_t)q0 + nq > (int64_t)e.B * e.max_q) {
+  if (nq < 0 || nq > ctx || ctx > e.max_ctx || q0 < 0) {
     if (threadIdx.x == 0 && t == 0) record_error(a.d_err, MKV_DEVERR_CTX);
     return;
   }
@@ -702,15 +745,17 @@ attn_ext_f32_kernel(KArgs a, ExtArgs e) {
 }
 
 // Log-sum-exp merge of the extend kernel's key-range partials: one wave per
-// (query token, query head) row, partials row * splits + s.
+// (query token, query head) row, tokens counted from q_indptr[0], partials
+// row * splits + s.
 template <int D, bool BF16>
 __global__ void __launch_bounds__(256) merge_ext_kernel(KArgs a, ExtArgs e) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t row = (int64_t)blockIdx.x * 4 + wave;
-  const int64_t tokens = min((int64_t)e.q_indptr[e.B], (int64_t)e.B * e.max_q);
-  if (row >= tokens * a.Hq) return;
-  merge_rows<D, BF16>(a, lane, row * e.splits, 1, e.splits, row);
+  const int64_t part0 = e.q_indptr[0];
+  const int64_t tokens = min((int64_t)e.q_indptr[e.B] - part0, (int64_t)e.B * e.max_q);
+  if (part0 < 0 || row >= tokens * a.Hq) return;
+  merge_rows<D, BF16>(a, lane, row * e.splits, 1, e.splits, part0 * a.Hq + row);
 }
 
 }  // namespace mkv

@@ -237,3 +237,44 @@ def test_extend_row_tiles(shape, chunks):
     ctx, nq = chunks
     got, ref, _, _ = _case(shape, ctx, nq, 104)
     assert_attention_close(got, ref, "bf16")
+
+
+@pytest.mark.parametrize("shape", [(28, 4, 128, "bf16"), (64, 2, 128, "bf16"), (8, 1, 256, "bf16"), (6, 2, 64, "bf16"),
+                                   (14, 2, 64, "f32"), (5, 1, 256, "f32")])
+@pytest.mark.parametrize("chunks", [
+    # (contexts, new tokens, max_q_len): key ranges in one piece (fewer than
+    # 512 keys), one chunk just past a tile and one of many rounds; and key
+    # ranges that are cut, the chunks' tokens within num_seqs * max_q_len
+    ([200, 150, 30], [70, 150, 5], 16),
+    ([90, 255], [2, 255], 1),
+    ([2000, 900, 1500], [20, 3, 1], 16),
+])
+@pytest.mark.parametrize("first", [0, 7])
+def test_extend_chunk_longer_than_max_q_len(shape, chunks, first):
+    """Every token of q_indptr is computed, whatever max_q_len said of the
+    chunks and wherever q_indptr starts, and rows outside it are left alone."""
+    Hq, Hkv, D, dt = shape
+    ctx, nq, max_q = chunks
+    batch = wl.decode_batch_from_contexts([c - 1 for c in ctx], wl.SplitMix64(105), extra_blocks=2)
+    desc = PoolDesc(1, Hkv, Hq, D, batch.num_blocks, dt)
+    host = normal(106, desc.shape, dt)
+    q_indptr = np.concatenate([[0], np.cumsum(nq)]).astype(np.int32)
+    total = int(q_indptr[-1])
+    q = normal(107, (first + total + 3, Hq, D), dt)
+    with DeviceKvPool(desc) as pool:
+        pool.write(host)
+        out = to_device(np.zeros_like(q))
+        pool.extend_attention(0, to_device(q), _i32(q_indptr + first), _i32(batch.block_indptr),
+                              _i32(batch.block_ids), _i32(batch.ctx_lens), max_q, max(ctx), out=out)
+        pool.check()
+        got = to_host(out)
+        # a chunk that starts before row 0 is reported, not read
+        pool.extend_attention(0, to_device(q), _i32(q_indptr - 2), _i32(batch.block_indptr), _i32(batch.block_ids),
+                              _i32(batch.ctx_lens), max_q, max(ctx), out=out)
+        with pytest.raises(DeviceIndexError) as ei:
+            pool.check()
+        assert ei.value.bits & dp.DEVERR_CTX
+    ref = orc.extend_attention(odesc(desc), host, 0, widen(q[first:first + total]), q_indptr, batch.block_indptr,
+                               batch.block_ids, batch.ctx_lens)
+    assert_attention_close(got[first:first + total], ref, dt)
+    assert not np.any(got[:first]) and not np.any(got[first + total:])
