@@ -94,10 +94,11 @@ __device__ __forceinline__ bool ext_tile(const ExtArgs &e, int Hkv, int &t, int 
 }
 
 // One row tile t of (KV head h, sequence of nq queries from token q0 over ctx
-// keys, its table at a.ids + tab0), key-range split sp.
+// keys, its table at a.ids + tab0), key-range split sp. odd_s (in LDS) becomes
+// 1 where an Inf or NaN was left out of the V tiles (extend_odd_values).
 template <int D, int W, int KB, int R>
 __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, int t, int h, int sp, int q0, int nq,
-                                            int ctx, int tab0, int part0) {
+                                            int ctx, int tab0, int part0, int &odd_s) {
   constexpr int NR = D / 32, NT = D / 16;
   constexpr int RB = D * 2;                           // LDS tile row: one head's K or V row
   constexpr int CPR = RB / 16;                        // 16-byte chunks per tile row
@@ -134,6 +135,7 @@ __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, in
   const int qlo = e.causal ? p0 + min(row0, rows - 1) / a.G : ctx - 1;
   const int qhi = e.causal ? p0 + min(row0 + 15, rows - 1) / a.G : ctx - 1;
   const int qhi_wg = e.causal ? p0 + (min(tile_rows * (t + 1), rows) - 1) / a.G : ctx - 1;
+  const int qlo_wg = e.causal ? p0 + tile_rows * t / a.G : ctx - 1;
   const int n = qhi_wg / kPageSize + 1;           // blocks the workgroup streams: keys 0..qhi_wg
   const int nw = min(n, qhi / kPageSize + 1);     // blocks this wave's rows see
   // Steps of KB blocks; with splits, this workgroup takes its share of them
@@ -198,17 +200,17 @@ __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, in
   constexpr bool kLean = LPL <= 4;
   __shared__ int32_t ids_s[kLean ? kExtIdCap : 1];
   const int kfirst = st0 * KB, kend = min(st1 * KB, n);
-  int fast = kLean && kend - kfirst <= kExtIdCap;
-  if (fast) {
-    int badl = 0;
+  int slow = !(kLean && kend - kfirst <= kExtIdCap);
+  if (tid == 0) odd_s = 0;
+  if (!slow) {
     const int32_t *tg = a.ids + tab0 + kfirst;
     for (int i = tid; i < kend - kfirst; i += 64 * W) {
       const int32_t id = tg[i];
-      badl |= (id < 0) | (id >= a.nblocks);
+      slow |= (id < 0) | (id >= a.nblocks);
       ids_s[i] = id;
     }
-    fast = !__syncthreads_or(badl);
   }
+  int fast = !__syncthreads_or(slow);
   fast = __builtin_amdgcn_readfirstlane(fast);
   // A wave past the step's chunks (head_dim 64 with 16 waves) loads the
   // step's last chunks again and does not store them: one load form, so the
@@ -279,7 +281,24 @@ __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, in
         // zeros (stale slots may hold any bit pattern, and p = 0 times NaN
         // would poison O); K rows there are masked in the scores instead.
         u32x4 val = ring[s][i];
-        if (kv && (((badr[s] >> kb) & 1) || kPageSize * (step * KB + kb) + row >= ctx)) val = u32x4{0u, 0u, 0u, 0u};
+        const int key = kPageSize * (step * KB + kb) + row;
+        if (kv && (((badr[s] >> kb) & 1) || key >= ctx)) val = u32x4{0u, 0u, 0u, 0u};
+        if (kv && key > qlo_wg) {
+          // Hidden from the tile's first row, with p = 0, and 0 times Inf or
+          // NaN is NaN: such values (exponent of all ones) are left out here
+          // and added to the rows that see them once the tile is done.
+          uint32_t odd = 0;
+#pragma unroll
+          for (int x = 0; x < 4; x++) odd |= (val[x] & 0x7f807f80u) + 0x00800080u;
+          if (odd & 0x80008000u) {
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+              const uint32_t one = (((val[x] & 0x7f807f80u) + 0x00800080u) >> 15) & 0x00010001u;
+              val[x] &= ~((one << 16) - one);
+            }
+            odd_s = 1;
+          }
+        }
         *reinterpret_cast<u32x4 *>(tiles[s & 1][kb][kv] + row * RB + ((cc ^ (kv ? ext_v_swz(row, CPR) : ext_k_swz(row, CPR))) << 4)) = val;
       }
     }
@@ -410,7 +429,7 @@ __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, in
   // Fast steps: [st0, fast_end), blocks below the workgroup's first query
   // position and below ctx (all keys visible to all its queries), with the
   // steps issued R - 1 ahead inside [kfirst, kend).
-  const int fb = e.causal ? min((p0 + tile_rows * t / a.G + 1) / kPageSize, ctx / kPageSize) : ctx / kPageSize;
+  const int fb = e.causal ? min((qlo_wg + 1) / kPageSize, ctx / kPageSize) : ctx / kPageSize;
   const int fast_end = fast ? max(st0, min(min(st1, fb / KB), kend / KB - (R - 1))) : st0;
   const std::integral_constant<bool, true> kFast;
   const std::integral_constant<bool, false> kGeneric;
@@ -450,6 +469,59 @@ __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, in
                                                           pack_bf16x2(st.O[nn][2] * f, st.O[nn][3] * f));
 }
 
+// The Inf and NaN values of V that row tile t left out, added to what it stored
+// for the rows that see their keys (a weight is positive, so the row becomes
+// Inf or NaN in that dim). Every key past the tile's first position is looked
+// at again; only chunks that hold such values come here. (Looking for them in
+// the masked blocks of a tile costs whole prompts 1-3% in bf16 and up to 4% in
+// f32: 12 of 20-200 tokens, 14 heads of 64: 18.2 -> 18.9 us.)
+template <int D, int THREADS, int KB, bool BF16>
+__device__ __forceinline__ void extend_odd_values(const KArgs &a, const ExtArgs &e, int tile_rows, int t, int h, int sp,
+                                                  int q0, int nq, int ctx, int tab0, int part0) {
+  const int rows = nq * a.G, r0 = tile_rows * t, r1 = min(rows, r0 + tile_rows), p0 = ctx - nq;
+  const int n = (p0 + (r1 - 1) / a.G) / kPageSize + 1;
+  const int steps = (n + KB - 1) / KB, sps = (steps + e.splits - 1) / e.splits;
+  const int key0 = max(p0 + r0 / a.G + 1, kPageSize * KB * min(sp * sps, steps));
+  const int key1 = min(ctx, kPageSize * min(KB * min((sp + 1) * sps, steps), n));
+#pragma unroll 1
+  for (int i = threadIdx.x; i < (r1 - r0) * (D / 4); i += THREADS) {
+    const int r = r0 + i / (D / 4), d = 4 * (i % (D / 4)), pos = r / a.G;
+    float add[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int key = key0; key < min(key1, p0 + pos + 1); key++) {
+      const int32_t blk = a.ids[tab0 + key / kPageSize];
+      if (blk < 0 || blk >= a.nblocks) continue;
+      const uint8_t *vp = a.v_plane + (int64_t)blk * a.block_bytes + (int64_t)(key % kPageSize) * a.row_bytes +
+                          (h * D + d) * (BF16 ? 2 : 4);
+      float x[4];
+      if constexpr (BF16) {
+        const uint2 v = *reinterpret_cast<const uint2 *>(vp);
+        x[0] = bf16_lo(v.x), x[1] = bf16_hi(v.x), x[2] = bf16_lo(v.y), x[3] = bf16_hi(v.y);
+      } else {
+        const f32x4 v = *reinterpret_cast<const f32x4 *>(vp);
+        x[0] = v[0], x[1] = v[1], x[2] = v[2], x[3] = v[3];
+      }
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+        if ((__float_as_uint(x[c]) & 0x7f800000u) == 0x7f800000u) add[c] += x[c];
+    }
+    const int64_t qrow = (int64_t)(q0 + pos) * a.Hq + h * a.G + (r - pos * a.G);
+    const int64_t prow = (qrow - (int64_t)part0 * a.Hq) * e.splits + sp;
+    const bool part = e.splits > 1 || e.partial;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      if (add[c] == 0.0f) continue;
+      if (part || !BF16) {
+        float *op = part ? a.ws_o + prow * D : reinterpret_cast<float *>(a.o) + qrow * D;
+        op[d + c] += add[c];
+      } else {
+        uint16_t *op = reinterpret_cast<uint16_t *>(a.o) + qrow * D + d + c;
+        *op = (uint16_t)f32_to_bf16_bits(__uint_as_float((uint32_t)*op << 16) + add[c]);
+      }
+    }
+  }
+}
+
 template <int D, int W, int KB, int R>
 // (Eight waves at head_dim <= 128: two workgroups per CU, 128 registers. The
 // upper bound keeps the scheduler from saving registers for a fifth wave per
@@ -464,7 +536,8 @@ attn_extend_kernel(KArgs, ExtArgs) {
   // loop costs head_dim 64 up to 5% (16 chunks of 5-24 tokens 32 -> 33.9 us),
   // 128 nothing, and 256 gains from the arguments not kept (10%).
   static_assert(sizeof(KArgs) % alignof(ExtArgs) == 0, "ExtArgs follows KArgs");
-  for (int round = 0;; round++) {
+  __shared__ int odd_s;
+  for (int round = 0, odd = 0;;) {
     typedef const __attribute__((address_space(4))) uint8_t const_u8;
     const_u8 *ka = (const_u8 *)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(ka));
@@ -495,9 +568,16 @@ attn_extend_kernel(KArgs, ExtArgs) {
       return;
     }
     const bool more = tile_rows * (tt + e.tiles) < rows;
-    extend_tile<D, W, KB, R>(a, e, (int)tt, h, sp, q0, nq, ctx, tab0, part0);
-    if (!more) return;
-    __syncthreads();  // the next round writes the LDS tiles and ids again
+    if (odd) {
+      extend_odd_values<D, 64 * W, KB, true>(a, e, 16 * e.row_waves, (int)tt, h, sp, q0, nq, ctx, tab0, part0);
+      odd = 0;
+    } else {
+      extend_tile<D, W, KB, R>(a, e, (int)tt, h, sp, q0, nq, ctx, tab0, part0, odd_s);
+      odd = __builtin_amdgcn_readfirstlane(odd_s);
+    }
+    if (!odd && !more) return;
+    __syncthreads();  // the tile is stored; the next round writes the LDS again
+    round += !odd;
   }
 }
 
@@ -603,6 +683,7 @@ attn_ext_f32_kernel(KArgs a, ExtArgs e) {
     }
     f32x4 kr[RING][NK], vr[RING][4][NH];
     bool badr[RING];
+    int odd = 0;  // this wave left an Inf or NaN of V out (extend_odd_values)
     auto issue = [&](f32x4 (&kd)[NK], f32x4 (&vd)[4][NH], bool &bad, int k) {
       const int32_t blk = table[min(k, n - 1)];  // past the end: the last block again, unused
       bad = blk < 0 || blk >= a.nblocks;
@@ -677,6 +758,25 @@ attn_ext_f32_kernel(KArgs a, ExtArgs e) {
           if (bad || key + i >= ctx)
 #pragma unroll
             for (int hh = 0; hh < NH; hh++) vd[i][hh] = f32x4{0.f, 0.f, 0.f, 0.f};
+        float zero[4] = {0.f, 0.f, 0.f, 0.f};  // NaN where a V value is Inf or NaN
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int hh = 0; hh < NH; hh++)
+#pragma unroll
+            for (int nn = 0; nn < 4; nn++) zero[nn] = fmaf(vd[i][hh][nn], 0.0f, zero[nn]);
+        if (__ballot(__isnanf((zero[0] + zero[1]) + (zero[2] + zero[3])))) {
+          // Where the tile's first row does not see the key, 0 times that
+          // would be NaN: left out here, added once the tile is stored.
+          odd = 1;
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int hh = 0; hh < NH; hh++)
+#pragma unroll
+              for (int nn = 0; nn < 4; nn++)
+                if (key + i > first && (__float_as_uint(vd[i][hh][nn]) & 0x7f800000u) == 0x7f800000u) vd[i][hh][nn] = 0.0f;
+        }
       }
 #pragma unroll
       for (int i = 0; i < 4; i++)
@@ -716,7 +816,7 @@ attn_ext_f32_kernel(KArgs a, ExtArgs e) {
           *reinterpret_cast<f32x4 *>(&part[wave][row][((16 * hh + 4 * g4 + i) ^ c16) * 4]) =
               f32x4{O[s][4 * hh][i], O[s][4 * hh + 1][i], O[s][4 * hh + 2][i], O[s][4 * hh + 3][i]};
     }
-    __syncthreads();
+    odd = __syncthreads_or(odd);
 #pragma unroll
     for (int x = 0; x < ROWS * CPR / (64 * NW); x++) {
       const int at = (int)threadIdx.x + 64 * NW * x;
@@ -740,7 +840,9 @@ attn_ext_f32_kernel(KArgs a, ExtArgs e) {
       *reinterpret_cast<f32x4 *>(static_cast<float *>(a.o) +
                                  ((int64_t)(q0 + pos) * a.Hq + h * a.G + (r - pos * a.G)) * D + 4 * cc) = acc * f;
     }
-    __syncthreads();  // the next round writes the partials again
+    __syncthreads();  // the rows are stored; the next round writes the partials again
+    if (odd)
+      extend_odd_values<D, 64 * NW, 1, false>(a, e, ROWS, r0 / ROWS, h, 0, q0, nq, ctx, tab0, 0);
   }
 }
 
@@ -809,6 +911,7 @@ extern "C" int mkv_extend_attention(mkv_pool *pool, int32_t layer, const void *d
     e.B = num_seqs;
     e.max_ctx = max_ctx_len;
     e.max_q = max_q_len;
+    e.splits = 1;
     return launch_ext_f32(p, a, e, hs);
   }
   if (!use_mfma) {  // per-token segments on the decode kernels

@@ -278,3 +278,46 @@ def test_extend_chunk_longer_than_max_q_len(shape, chunks, first):
                                batch.block_ids, batch.ctx_lens)
     assert_attention_close(got[first:first + total], ref, dt)
     assert not np.any(got[:first]) and not np.any(got[first + total:])
+
+
+@pytest.mark.parametrize("shape", [(28, 4, 128, "bf16"), (64, 2, 128, "bf16"), (8, 1, 256, "bf16"), (3, 3, 64, "bf16"),
+                                   (14, 2, 64, "f32"), (2, 1, 128, "f32"), (5, 1, 256, "f32")])
+@pytest.mark.parametrize("chunks", [
+    ([70, 33, 200], [70, 20, 190]),   # whole prompts and chunks, key ranges in one piece
+    ([2000, 600, 900], [20, 3, 40]),  # bf16: key ranges that are cut
+])
+def test_extend_hidden_values_that_are_not_finite(shape, chunks):
+    """An Inf or NaN in a token's V row reaches the queries from that token on,
+    in its dims alone: a query before it has weight 0 there, not 0 * Inf."""
+    Hq, Hkv, D, dt = shape
+    ctx, nq = chunks
+    batch = wl.decode_batch_from_contexts([c - 1 for c in ctx], wl.SplitMix64(108), extra_blocks=2)
+    desc = PoolDesc(1, Hkv, Hq, D, batch.num_blocks, dt)
+    host = normal(109, desc.shape, dt)
+    inf, nan = (np.inf, np.nan) if dt == "f32" else (0x7F80, 0x7FC1)
+    ninf = -np.inf if dt == "f32" else 0xFF80
+
+    def v_row(b, pos):
+        return host[0, 1, batch.block_ids[batch.block_indptr[b] + pos // 16], pos % 16]
+
+    v_row(0, ctx[0] - 5)[:, 3] = inf
+    v_row(0, ctx[0] - 2)[:, 3] = ninf          # Inf - Inf from here on
+    v_row(0, ctx[0] - 9)[Hkv - 1, D - 1] = nan
+    v_row(1, ctx[1] - nq[1] + 1)[0, 8:17] = ninf
+    v_row(2, ctx[2] - 1)[:] = nan              # the last query alone
+    v_row(2, ctx[2] - nq[2])[0, 0] = inf       # every query of the chunk
+    q_indptr = np.concatenate([[0], np.cumsum(nq)]).astype(np.int32)
+    q = normal(110, (int(q_indptr[-1]), Hq, D), dt)
+    with DeviceKvPool(desc) as pool:
+        pool.write(host)
+        got = widen(to_host(pool.extend_attention(0, to_device(q), _i32(q_indptr), _i32(batch.block_indptr),
+                                                  _i32(batch.block_ids), _i32(batch.ctx_lens), max(nq), max(ctx))))
+        pool.check()
+    ref = orc.extend_attention(odesc(desc), host, 0, widen(q), q_indptr, batch.block_indptr, batch.block_ids,
+                               batch.ctx_lens)
+    odd = ~np.isfinite(ref)
+    assert odd.any() and not odd.all()
+    np.testing.assert_array_equal(got[odd], ref[odd])
+    assert np.isfinite(got[~odd]).all()
+    got, ref = np.where(odd, 0, got).astype(np.float32), np.where(odd, 0, ref).astype(np.float32)
+    assert_attention_close(got if dt == "f32" else orc.f32_to_bf16(got), ref, dt)
