@@ -196,11 +196,12 @@ __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, in
   // plane per wave, so a load is a wave-uniform base (block id, plane) plus a
   // lane offset (row, chunk, head) fixed for the whole launch.
   // (More than four loads per lane and step would hold more registers than the
-  // lean path saves: those launches keep the generic path.)
-  constexpr bool kLean = LPL <= 4;
-  __shared__ int32_t ids_s[kLean ? kExtIdCap : 1];
+  // lean path saves, and without it head_dim 256 takes twice the time: one
+  // token after 8k 56 us with 8 waves, 116 with 4, whose 8 loads rule it out.)
+  static_assert(LPL <= 4, "every instantiation has the lean path");
+  __shared__ int32_t ids_s[kExtIdCap];
   const int kfirst = st0 * KB, kend = min(st1 * KB, n);
-  int slow = !(kLean && kend - kfirst <= kExtIdCap);
+  int slow = kend - kfirst > kExtIdCap;
   if (tid == 0) odd_s = 0;
   if (!slow) {
     const int32_t *tg = a.ids + tab0 + kfirst;
@@ -527,7 +528,7 @@ template <int D, int W, int KB, int R>
 // upper bound keeps the scheduler from saving registers for a fifth wave per
 // SIMD, which serialised the V reads: 31.5 -> 34.6 us for one token after 8k
 // at head_dim 64.)
-__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 128 ? (W == 4 ? 2 : 4) : W / 4, D <= 128 ? 4 : W / 4)))
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256 || W == 4 ? 2 : 4, D == 256 ? 2 : 4)))
 attn_extend_kernel(KArgs, ExtArgs) {
   // One tile per workgroup; a chunk longer than max_q_len takes further rounds.
   // Each round reads the arguments again, through a pointer that the compiler
@@ -976,15 +977,15 @@ extern "C" int mkv_extend_attention_host(mkv_pool *pool, int32_t layer, const vo
   return rc ? rc : rr;
 }
 
-// The extend kernel's instantiation for head_dim D and W waves (4, 8 or 16; 4
-// or 8 at head_dim 256: 16 waves cap the registers at 128, and its state then
-// spills).
+// The extend kernel's instantiation for head_dim D and W waves (4, 8 or 16; 8
+// at head_dim 256: 16 waves cap the registers at 128, and its state then
+// spills; 4 waves would carry 8 loads a lane and step).
 const void *mkv::ext_kernel(int D, int W) {
 #define MKV_EXT_FN(DD, WW) reinterpret_cast<const void *>(&attn_extend_kernel<DD, WW, kExtKB, kExtR>)
   switch (D) {
     case 64: return W == 4 ? MKV_EXT_FN(64, 4) : W == 8 ? MKV_EXT_FN(64, 8) : MKV_EXT_FN(64, 16);
     case 128: return W == 4 ? MKV_EXT_FN(128, 4) : W == 8 ? MKV_EXT_FN(128, 8) : MKV_EXT_FN(128, 16);
-    default: return W == 4 ? MKV_EXT_FN(256, 4) : MKV_EXT_FN(256, 8);
+    default: return MKV_EXT_FN(256, 8);
   }
 #undef MKV_EXT_FN
 }
@@ -1020,13 +1021,12 @@ int mkv::launch_ext_tiles(Pool *p, KArgs &a, ExtArgs &e, int split_cap, hipStrea
   const int64_t num_seqs = e.B, max_q_len = e.max_q, max_ctx_len = e.max_ctx;
   if (((max_q_len + 15) / 16 * g.Hq * num_seqs) * split_cap + 8 > INT32_MAX)
     return set_error(MKV_ERR_INVALID_ARGUMENT, "grid too large");
-  // Waves per workgroup: enough for the longest chunk's rows, at most 16 (8 at
-  // head_dim 256 and beside a decode launch), so that a K/V tile in LDS serves
-  // as many rows as it can; at least 4, since waves past the last row still
-  // share the loads.
+  // Waves per workgroup: enough for the longest chunk's rows, at most 16 (8
+  // beside a decode launch), so that a K/V tile in LDS serves as many rows as
+  // it can; at least 4, since waves past the last row still share the loads.
+  // Always 8 at head_dim 256 (ext_kernel).
   const int64_t rows_max = max_q_len * G;
-  const int most = beside || g.D == 256 ? 8 : 16;
-  const int W = rows_max <= 64 ? 4 : rows_max <= 128 ? 8 : most;
+  const int W = g.D == 256 ? 8 : rows_max <= 64 ? 4 : rows_max <= 128 || beside ? 8 : 16;
   const void *fn = ext_kernel(g.D, W);
   const int64_t rows = (int64_t)num_seqs * max_q_len * g.Hq;  // bounds the (token, query head) rows
   // Slots = resident workgroups per CU of this instantiation (occupancy query,
@@ -1055,7 +1055,7 @@ int mkv::launch_ext_tiles(Pool *p, KArgs &a, ExtArgs &e, int split_cap, hipStrea
     // No split is faster than the K/V bytes (of contexts of 0.6 of the longest).
     const double kv_cost = kExtCostPerUs * 0.6 * (double)num_seqs * (double)max_ctx_len * 2 * (double)g.row_bytes / 5.5e6;
     const int64_t most_splits = std::max<int64_t>(1, std::min<int64_t>(split_cap, steps_max / 8));
-    for (int k = W; 2 * k > W; k--) {
+    for (int k = (int)std::min<int64_t>(W, (rows_max + 15) / 16); 2 * k > W || (k > 0 && 16 * k >= rows_max); k--) {
       const int64_t wgs = (rows_max + 16 * k - 1) / (16 * k) * g.Hkv * num_seqs;
       for (int64_t sp = 1; sp <= (wgs < slots ? most_splits : 1); sp++) {
         const double x = (double)(wgs * sp) / (double)slots;
