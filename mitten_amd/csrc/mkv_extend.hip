@@ -201,7 +201,13 @@ __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, in
   static_assert(LPL <= 4, "every instantiation has the lean path");
   __shared__ int32_t ids_s[kExtIdCap];
   const int kfirst = st0 * KB, kend = min(st1 * KB, n);
-  int slow = kend - kfirst > kExtIdCap;
+  // Fast steps: [st0, fast_end), blocks below the workgroup's first query
+  // position and below ctx (all keys visible to all its queries), with the
+  // steps issued R - 1 ahead inside [kfirst, kend). A tile without any stages
+  // no ids: its first loads would wait for them.
+  const int fb = e.causal ? min((qlo_wg + 1) / kPageSize, ctx / kPageSize) : ctx / kPageSize;
+  int fast_end = min(min(st1, fb / KB), kend / KB - (R - 1));
+  int slow = fast_end <= st0 || kend - kfirst > kExtIdCap;
   if (tid == 0) odd_s = 0;
   if (!slow) {
     const int32_t *tg = a.ids + tab0 + kfirst;
@@ -211,8 +217,7 @@ __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, in
       ids_s[i] = id;
     }
   }
-  int fast = !__syncthreads_or(slow);
-  fast = __builtin_amdgcn_readfirstlane(fast);
+  if (__builtin_amdgcn_readfirstlane(__syncthreads_or(slow))) fast_end = st0;
   // A wave past the step's chunks (head_dim 64 with 16 waves) loads the
   // step's last chunks again and does not store them: one load form, so the
   // compiler's in-order load counting stays exact.
@@ -427,11 +432,6 @@ __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, in
 
 #pragma unroll
   for (int s = 0; s < R - 1; s++) issue(ring[s], badr[s], st0 + s);
-  // Fast steps: [st0, fast_end), blocks below the workgroup's first query
-  // position and below ctx (all keys visible to all its queries), with the
-  // steps issued R - 1 ahead inside [kfirst, kend).
-  const int fb = e.causal ? min((qlo_wg + 1) / kPageSize, ctx / kPageSize) : ctx / kPageSize;
-  const int fast_end = fast ? max(st0, min(min(st1, fb / KB), kend / KB - (R - 1))) : st0;
   const std::integral_constant<bool, true> kFast;
   const std::integral_constant<bool, false> kGeneric;
   int k0 = st0;
@@ -549,12 +549,14 @@ attn_extend_kernel(KArgs, ExtArgs) {
     const const_i32 *ctx_lens = (const const_i32 *)e.ctx;
     int t, h, b, sp;
     if (!ext_tile(e, a.Hkv, t, h, b, sp)) return;
-    const bool virt = e.q_indptr == nullptr;  // one sequence; the host checked its table length
-    const int q0 = virt ? 0 : q_indptr[b], nq = virt ? e.v_nq : q_indptr[b + 1] - q0;
+    // The sequence's metadata at once (one round trip, not one per check).
+    int q0 = 0, nq = e.v_nq, ctx = e.v_ctx, tab0 = 0, tab1 = 0;  // one sequence, its table length checked by the host
+    const bool virt = e.q_indptr == nullptr;
+    if (!virt) q0 = q_indptr[b], nq = q_indptr[b + 1], ctx = ctx_lens[b], tab0 = indptr[b], tab1 = indptr[b + 1];
+    nq -= q0;
     const int64_t rows = (int64_t)nq * a.G, tile_rows = 16 * e.row_waves;
     const int64_t tt = t + (int64_t)e.tiles * round;
     if (nq <= 0 || tile_rows * tt >= rows) return;
-    const int ctx = virt ? e.v_ctx : ctx_lens[b];
     // Partial rows exist for num_seqs * max_q_len tokens from q_indptr[0] on.
     const bool parts = e.splits > 1 || e.partial;
     const int part0 = parts && !virt ? q_indptr[0] : 0;
@@ -563,8 +565,7 @@ attn_extend_kernel(KArgs, ExtArgs) {
       if (threadIdx.x == 0 && t == 0) record_error(a.d_err, MKV_DEVERR_CTX);
       return;
     }
-    const int tab0 = virt ? 0 : indptr[b], nbt = (ctx + kPageSize - 1) / kPageSize;
-    if (!virt && (tab0 < 0 || indptr[b + 1] - tab0 < nbt)) {
+    if (!virt && (tab0 < 0 || tab1 - tab0 < (ctx + kPageSize - 1) / kPageSize)) {
       if (threadIdx.x == 0 && t == 0) record_error(a.d_err, MKV_DEVERR_TABLE);
       return;
     }
