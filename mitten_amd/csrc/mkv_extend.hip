@@ -1008,6 +1008,52 @@ int mkv::ext_resident_per_cu(Pool *p, const void *fn, int W) {
   return per_cu;
 }
 
+// What a launch of the extend kernel takes, in microseconds, by its waves per
+// workgroup (4, 8, 16), row waves per tile, key-range splits and size: the
+// rounds of resident workgroups times what one of them takes. The constants,
+// one set per head_dim, were fitted to the device times of 921 calls (1-128
+// sequences of 1-2,048 tokens over 0-8k, 21 head shapes, equal and ragged) at
+// every choice of the three, then moved to where the choice by them comes
+// closest to the best of each call's table: 3% from the best of the choices it
+// may make, on average. The rule before it took as many waves as the rows fill
+// and constants of head_dim 128 throughout: 12% slower on average, and 132 of
+// the calls more than 3% slower than before there were row tiles (8 heads on 4
+// of 64, 12 prompts beside one chunk after 6k: 117 us, 67 now; 8 heads on one
+// of 256, a 2,048-token prompt: 82 us, 59 now); 40 of them still are.
+struct ExtCost {
+  double step[3], step_row[3];  // a step (32 keys) of one workgroup alone: + per row wave
+  double cu[3], cu_row;         // a step's share of the CU where several are resident
+  double start;                 // a workgroup's first loads and last stores, once per round
+  double launch, tail, tail_split;
+  double merge, merge_value;    // the merge launch; a partial value written and read
+};
+static const ExtCost kExtCost[3] = {
+    {{.31, .31, .45}, {.011, .012, .011}, {.13, .19, .016}, .0084, 1.1, 4.6, .83, .44, 2.5, 2.3e-6},
+    {{.32, .48, .31}, {.020, .029, .025}, {.18, .16, .18}, .025, 3.6, 5.2, .26, .10, 1.5, 1.8e-6},
+    {{0, .68, 0}, {0, .095, 0}, {0, .033, 0}, .019, 4.4, 2.8, .60, .78, 5.9, 1.2e-6},  // 8 waves only
+};
+
+// wgs: workgroups, splits included, of which per_cu are resident on each of cus
+// CUs; steps: of the longest; share: mean keys of a tile over the longest (whole
+// prompts' tiles shrink from longest to shortest, so a started round fills up,
+// less so where splits tie them to an XCD; above kExtEqualShare they count as
+// equal and rounds as whole ones); values: partial values, splits included.
+constexpr double kExtEqualShare = 0.85;
+static double ext_cost_us(const ExtCost &c, int W, int row_waves, double wgs, double cus, int per_cu, double steps,
+                          double share, bool split, bool equal, double values) {
+  const int w = W == 4 ? 0 : W == 8 ? 1 : 2;
+  const double resident = std::min<double>(per_cu, std::max(1.0, std::ceil(wgs / cus)));
+  const double x = wgs / (cus * resident), y = x * share;
+  const double step = std::max(c.step[w] + c.step_row[w] * row_waves, resident * (c.cu[w] + c.cu_row * row_waves));
+  const double whole = equal ? (x <= 1 ? 1 : x <= 4 ? std::ceil(x) : x + 0.5) : std::max(1.0, x);
+  double rounds = whole;
+  if (share <= kExtEqualShare || !equal) {
+    const double f = std::min(1.0, y);
+    rounds = split ? (x <= 1 ? 1 : std::max(1.0, y + c.tail_split)) : std::max(1.0, y + c.tail * f * f);
+  }
+  return c.launch + rounds * steps * step + whole * c.start + (split ? c.merge : 0) + c.merge_value * values;
+}
+
 // MFMA query tiles of the extend kernel for e (B, max_q, max_ctx, causal,
 // partial and the sequence arguments set): picks the instantiation and the
 // key-range split (at most split_cap), grows the pool workspace when
@@ -1022,56 +1068,54 @@ int mkv::launch_ext_tiles(Pool *p, KArgs &a, ExtArgs &e, int split_cap, hipStrea
   const int64_t num_seqs = e.B, max_q_len = e.max_q, max_ctx_len = e.max_ctx;
   if (((max_q_len + 15) / 16 * g.Hq * num_seqs) * split_cap + 8 > INT32_MAX)
     return set_error(MKV_ERR_INVALID_ARGUMENT, "grid too large");
-  // Waves per workgroup: enough for the longest chunk's rows, at most 16 (8
-  // beside a decode launch), so that a K/V tile in LDS serves as many rows as
-  // it can; at least 4, since waves past the last row still share the loads.
-  // Always 8 at head_dim 256 (ext_kernel).
-  const int64_t rows_max = max_q_len * G;
-  const int W = g.D == 256 ? 8 : rows_max <= 64 ? 4 : rows_max <= 128 || beside ? 8 : 16;
-  const void *fn = ext_kernel(g.D, W);
+  const int64_t rows_max = max_q_len * G, row_waves_max = (rows_max + 15) / 16;
   const int64_t rows = (int64_t)num_seqs * max_q_len * g.Hq;  // bounds the (token, query head) rows
-  // Slots = resident workgroups per CU of this instantiation (occupancy query,
-  // once per pool) x CUs; one per CU beside a decode launch.
-  const int per_cu = ext_resident_per_cu(p, fn, W);
-  const int cus = device_cus(p);
-  const int64_t slots = per_cu > 0 && cus > 0 ? (beside ? 1 : (int64_t)per_cu) * cus : 0;
   const int64_t steps_max = ((int64_t)(max_ctx_len + kPageSize - 1) / kPageSize + kExtKB - 1) / kExtKB;
-  // Row waves per tile and key-range splits: the pair whose rounds of resident
-  // workgroups take least. A step of a workgroup costs kExtStepWaves + its row
-  // waves (8 x 512 after 4k: two rounds of 16 row waves 317 us, of 14 300 us),
-  // so full tiles are best until a smaller one saves part of a round. A key
-  // range splits where the launch leaves resident slots empty (short chunks
-  // over long contexts: one workgroup per (sequence, KV head) would stream a
-  // whole context), in at most split_cap of at least 8 steps apiece; the f32
-  // partials go to the pool-owned workspace and a second launch merges them
-  // (kExtMergeCost, and each partial's write and read).
-  constexpr double kExtStepWaves = 22, kExtMergeCost = 150, kExtCostPerUs = 36;
-  // Mean keys of a tile over the longest: whole prompts' tiles shrink from
-  // longest to shortest and fill a started round, equal ones do not.
   const double share = e.causal ? 1.0 - 0.5 * (double)max_q_len / (double)max_ctx_len : 1.0;
+  const int cus = device_cus(p);
+  const ExtCost &ec = kExtCost[g.D == 64 ? 0 : g.D == 128 ? 1 : 2];
+  // Waves per workgroup (8 at head_dim 256, at most 8 beside a decode launch;
+  // waves past the tile's rows share the loads), row waves per tile (half of
+  // them or more, or what the rows fill) and key-range splits: the least cost.
+  // A key range splits only where the launch leaves resident slots empty (short
+  // chunks over long contexts), in at most split_cap of at least 8 steps apiece
+  // and into two rounds; the f32 partials go to the pool-owned workspace and a
+  // second launch merges them. The cost is that of num_seqs sequences of the largest sizes, and with
+  // a fourth of the weight that of a fifth as many (in powers, no logarithm):
+  // lengths differ, and what a fuller launch wins little by can cost a ragged
+  // one much (14 heads on 2 of 64, 40 short prompts beside one chunk after 8k:
+  // 112 us without, 65 with).
+  int W = g.D == 256 ? 8 : row_waves_max <= 4 ? 4 : row_waves_max <= 8 || beside ? 8 : 16;
   e.splits = 1;
-  e.row_waves = W;
-  if (slots > 0) {
-    double best = INFINITY;
-    // No split is faster than the K/V bytes (of contexts of 0.6 of the longest).
-    const double kv_cost = kExtCostPerUs * 0.6 * (double)num_seqs * (double)max_ctx_len * 2 * (double)g.row_bytes / 5.5e6;
+  e.row_waves = (int32_t)std::min<int64_t>(W, row_waves_max);
+  double best = INFINITY;
+  for (int w = g.D == 256 ? 8 : 4; w <= (beside || g.D == 256 ? 8 : 16); w *= 2) {
+    if (g.D < 256 && w > 4 && row_waves_max < w / 4) break;
+    // Resident workgroups per CU of this instantiation (occupancy query, once
+    // per pool); one beside a decode launch.
+    int per_cu = ext_resident_per_cu(p, ext_kernel(g.D, w), w);
+    if (per_cu < 1 || cus < 1) continue;
+    if (beside) per_cu = 1;
     const int64_t most_splits = std::max<int64_t>(1, std::min<int64_t>(split_cap, steps_max / 8));
-    for (int k = (int)std::min<int64_t>(W, (rows_max + 15) / 16); 2 * k > W || (k > 0 && 16 * k >= rows_max); k--) {
-      const int64_t wgs = (rows_max + 16 * k - 1) / (16 * k) * g.Hkv * num_seqs;
-      for (int64_t sp = 1; sp <= (wgs < slots ? most_splits : 1); sp++) {
-        const double x = (double)(wgs * sp) / (double)slots;
-        const double rounds = share > 0.85 ? (x <= 4 ? std::ceil(x) : x + 0.5) : std::max(1.0, x * share + 0.25);
-        double cost = rounds * (double)((steps_max + sp - 1) / sp) * (kExtStepWaves + k);
-        cost = std::max(cost, kv_cost);
-        if (sp > 1) cost += kExtMergeCost + kExtCostPerUs * ((double)rows * sp * g.D * 8 / 5e6);
+    for (int64_t k = std::min<int64_t>(w, row_waves_max), least = row_waves_max < w ? k : w / 2; k >= least; k--) {
+      const int64_t wgs = (row_waves_max + k - 1) / k * g.Hkv * num_seqs;
+      const int64_t slots = (int64_t)per_cu * cus, most = wgs < slots ? std::min(most_splits, 2 * slots / wgs) : 1;
+      for (int64_t sp = 1; sp <= most; sp++) {
+        const double steps = (double)((steps_max + sp - 1) / sp), n = (double)(wgs * sp);
+        const double values = sp > 1 || e.partial ? (double)(rows * sp * g.D) : 0;
+        const double all = ext_cost_us(ec, w, (int)k, n, cus, per_cu, steps, share, sp > 1, true, values);
+        const double few = ext_cost_us(ec, w, (int)k, 0.2 * n, cus, per_cu, steps, share, sp > 1, false, 0.2 * values);
+        const double cost = all * all * all * all * few;
         if (cost < best) {
           best = cost;
-          e.row_waves = k;
+          W = w;
+          e.row_waves = (int32_t)k;
           e.splits = (int32_t)sp;
         }
       }
     }
   }
+  const void *fn = ext_kernel(g.D, W);
   const int64_t tiles = (rows_max + 16 * e.row_waves - 1) / (16 * e.row_waves);
   const int64_t per_split = tiles * g.Hkv * num_seqs;  // (tile, KV head, sequence) workgroups
   if (e.splits > 1 || e.partial) {
@@ -1092,7 +1136,7 @@ int mkv::launch_ext_tiles(Pool *p, KArgs &a, ExtArgs &e, int split_cap, hipStrea
   const int64_t total = per_split * e.splits;  // linear index -> (tile, KV head, sequence, split), by XCD
   e.tiles = (int32_t)tiles;
   e.per_xcd = (int32_t)((total + 7) / 8);
-  e.spread = share <= 0.85 && e.splits == 1;
+  e.spread = share <= kExtEqualShare && e.splits == 1;
   const dim3 grid((unsigned)(8 * (int64_t)e.per_xcd)), block(64 * W);
   void *args[] = {&a, &e};
   MKV_CHECK_HIP(hipLaunchKernel(fn, grid, block, args, 0, hs));
