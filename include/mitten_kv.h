@@ -407,10 +407,13 @@ MKV_API int mkv_decode_step_shared_prefix(mkv_pool *pool, const mkv_decode_plan 
  * per query token.
  * When the bf16 tiles would leave the device's resident workgroup slots
  * empty (few short chunks over long contexts, at most 16 query heads per KV
- * head), each key range is split in up to 4 and the f32 partials are merged by a second launch; they use the
- * pool-owned workspace shared with mkv_decode_attention (grown on demand:
- * that call synchronises the stream once, and such calls on one pool must
- * not run concurrently on different streams).
+ * head), each key range is split in up to 4 and the f32 partials are merged by
+ * a second launch; they use the pool-owned workspace shared with
+ * mkv_decode_attention (grown on demand: that call synchronises the stream
+ * once, or goes unsplit where the stream is being captured; a captured call
+ * keeps the workspace it saw, so no larger call may follow on the pool while
+ * its graph is replayed; and such calls on one pool must not run concurrently
+ * on different streams).
  * Flags: MKV_ATTN_ZERO_SINK.
  * Replaces the seq_q > 1 path of inference-model-qwen/src/model.rs:410-416
  * with its causal mask (model.rs:542-555), for the chunks scheduled by

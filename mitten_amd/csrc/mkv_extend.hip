@@ -1085,42 +1085,55 @@ int mkv::launch_ext_tiles(Pool *p, KArgs &a, ExtArgs &e, int split_cap, hipStrea
   // lengths differ, and what a fuller launch wins little by can cost a ragged
   // one much (14 heads on 2 of 64, 40 short prompts beside one chunk after 8k:
   // 112 us without, 65 with).
-  int W = g.D == 256 ? 8 : row_waves_max <= 4 ? 4 : row_waves_max <= 8 || beside ? 8 : 16;
-  e.splits = 1;
-  e.row_waves = (int32_t)std::min<int64_t>(W, row_waves_max);
-  double best = INFINITY;
-  for (int w = g.D == 256 ? 8 : 4; w <= (beside || g.D == 256 ? 8 : 16); w *= 2) {
-    if (g.D < 256 && w > 4 && row_waves_max < w / 4) break;
-    // Resident workgroups per CU of this instantiation (occupancy query, once
-    // per pool); one beside a decode launch.
-    int per_cu = ext_resident_per_cu(p, ext_kernel(g.D, w), w);
-    if (per_cu < 1 || cus < 1) continue;
-    if (beside) per_cu = 1;
-    const int64_t most_splits = std::max<int64_t>(1, std::min<int64_t>(split_cap, steps_max / 8));
-    for (int64_t k = std::min<int64_t>(w, row_waves_max), least = row_waves_max < w ? k : w / 2; k >= least; k--) {
-      const int64_t wgs = (row_waves_max + k - 1) / k * g.Hkv * num_seqs;
-      const int64_t slots = (int64_t)per_cu * cus, most = wgs < slots ? std::min(most_splits, 2 * slots / wgs) : 1;
-      for (int64_t sp = 1; sp <= most; sp++) {
-        const double steps = (double)((steps_max + sp - 1) / sp), n = (double)(wgs * sp);
-        const double values = sp > 1 || e.partial ? (double)(rows * sp * g.D) : 0;
-        const double all = ext_cost_us(ec, w, (int)k, n, cus, per_cu, steps, share, sp > 1, true, values);
-        const double few = ext_cost_us(ec, w, (int)k, 0.2 * n, cus, per_cu, steps, share, sp > 1, false, 0.2 * values);
-        const double cost = all * all * all * all * few;
-        if (cost < best) {
-          best = cost;
-          W = w;
-          e.row_waves = (int32_t)k;
-          e.splits = (int32_t)sp;
+  int W = 0;
+  auto choose = [&](int cap) {
+    W = g.D == 256 ? 8 : row_waves_max <= 4 ? 4 : row_waves_max <= 8 || beside ? 8 : 16;
+    e.splits = 1;
+    e.row_waves = (int32_t)std::min<int64_t>(W, row_waves_max);
+    double best = INFINITY;
+    for (int w = g.D == 256 ? 8 : 4; w <= (beside || g.D == 256 ? 8 : 16); w *= 2) {
+      if (g.D < 256 && w > 4 && row_waves_max < w / 4) break;
+      // Resident workgroups per CU of this instantiation (occupancy query, once
+      // per pool); one beside a decode launch.
+      int per_cu = ext_resident_per_cu(p, ext_kernel(g.D, w), w);
+      if (per_cu < 1 || cus < 1) continue;
+      if (beside) per_cu = 1;
+      const int64_t most_splits = std::max<int64_t>(1, std::min<int64_t>(cap, steps_max / 8));
+      for (int64_t k = std::min<int64_t>(w, row_waves_max), least = row_waves_max < w ? k : w / 2; k >= least; k--) {
+        const int64_t wgs = (row_waves_max + k - 1) / k * g.Hkv * num_seqs;
+        const int64_t slots = (int64_t)per_cu * cus, most = wgs < slots ? std::min(most_splits, 2 * slots / wgs) : 1;
+        for (int64_t sp = 1; sp <= most; sp++) {
+          const double steps = (double)((steps_max + sp - 1) / sp), n = (double)(wgs * sp);
+          const double values = sp > 1 || e.partial ? (double)(rows * sp * g.D) : 0;
+          const double all = ext_cost_us(ec, w, (int)k, n, cus, per_cu, steps, share, sp > 1, true, values);
+          const double few = ext_cost_us(ec, w, (int)k, 0.2 * n, cus, per_cu, steps, share, sp > 1, false, 0.2 * values);
+          const double cost = all * all * all * all * few;
+          if (cost < best) {
+            best = cost;
+            W = w;
+            e.row_waves = (int32_t)k;
+            e.splits = (int32_t)sp;
+          }
         }
       }
+    }
+  };
+  choose(split_cap);
+  const uint64_t ml_bytes = ((uint64_t)rows * e.splits * 8 + 255) / 256 * 256;
+  uint64_t need = e.splits > 1 || e.partial ? ml_bytes + (uint64_t)rows * e.splits * g.D * 4 : 0;
+  if (need > p->ws_bytes && !e.partial) {
+    // The workspace cannot grow while the stream is captured: unsplit then.
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(hs, &cs) != hipSuccess) (void)hipGetLastError();
+    if (cs != hipStreamCaptureStatusNone) {
+      choose(1);
+      need = 0;
     }
   }
   const void *fn = ext_kernel(g.D, W);
   const int64_t tiles = (rows_max + 16 * e.row_waves - 1) / (16 * e.row_waves);
   const int64_t per_split = tiles * g.Hkv * num_seqs;  // (tile, KV head, sequence) workgroups
-  if (e.splits > 1 || e.partial) {
-    const uint64_t ml_bytes = ((uint64_t)rows * e.splits * 8 + 255) / 256 * 256;
-    const uint64_t need = ml_bytes + (uint64_t)rows * e.splits * g.D * 4;
+  if (need) {
     if (p->ws_bytes < need) {
       const uint64_t cap = std::max<uint64_t>(need, p->ws_bytes + p->ws_bytes / 2);
       MKV_CHECK_HIP(hipStreamSynchronize(hs));  // earlier launches may read the old buffer

@@ -321,3 +321,37 @@ def test_extend_hidden_values_that_are_not_finite(shape, chunks):
     assert np.isfinite(got[~odd]).all()
     got, ref = np.where(odd, 0, got).astype(np.float32), np.where(odd, 0, ref).astype(np.float32)
     assert_attention_close(got if dt == "f32" else orc.f32_to_bf16(got), ref, dt)
+
+
+def test_extend_captured_before_the_workspace_has_room():
+    """A call whose key ranges would be split, captured on a pool whose
+    workspace was never grown: unsplit, and every replay equals the oracle, with
+    the split call of the same sizes (which grows the workspace) in between."""
+    import torch
+
+    Hq, Hkv, D = SHAPES["qwen7b"]
+    ctx, nq = [2000, 700], [16, 5]
+    batch = wl.decode_batch_from_contexts([c - 1 for c in ctx], wl.SplitMix64(111), extra_blocks=2)
+    desc = PoolDesc(1, Hkv, Hq, D, batch.num_blocks, "bf16")
+    host = normal(112, desc.shape, "bf16")
+    q_indptr = np.concatenate([[0], np.cumsum(nq)]).astype(np.int32)
+    q = normal(113, (int(q_indptr[-1]), Hq, D), "bf16")
+    ref = orc.extend_attention(odesc(desc), host, 0, widen(q), q_indptr, batch.block_indptr, batch.block_ids,
+                               batch.ctx_lens)
+    with DeviceKvPool(desc) as pool:
+        pool.write(host)
+        args = (to_device(q), _i32(q_indptr), _i32(batch.block_indptr), _i32(batch.block_ids), _i32(batch.ctx_lens),
+                max(nq), max(ctx))
+        out, eager = torch.empty_like(args[0]), torch.empty_like(args[0])
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            pool.extend_attention(0, *args, out=out)
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert_attention_close(to_host(out), ref, "bf16")
+            pool.extend_attention(0, *args, out=eager)
+            assert_attention_close(to_host(eager), ref, "bf16")
+        pool.check()
