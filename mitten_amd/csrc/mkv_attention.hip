@@ -605,10 +605,12 @@ __global__ void __launch_bounds__(256) attn_split_kernel(KArgs a, SplitArgs sp) 
 }
 
 // Extend attention on the decode kernels' per-sequence segments, for pools
-// the extend kernels do not take (head_dim 32, or the MKV_ATTN_FORCE_VALU flag): query token t of sequence b, at position p,
-// is decode attention over keys 0..p through b's block table, with q and o
-// rows addressed by t (a virtual sequence per token). One unit per
-// (token, KV head, query-head chunk), whole context, final stores.
+// the extend kernels do not take (head_dim 32, or the MKV_ATTN_FORCE_VALU
+// flag): query token t of sequence b, at position p, is decode attention over
+// keys 0..p through b's block table, with q and o rows addressed by t (a
+// virtual sequence per token). One unit per (token, KV head, query-head
+// chunk), whole context, final stores. Never on MFMA (the dispatch's third
+// argument).
 struct ExtSplitArgs {
   const int32_t *q_indptr;  // [B+1]
   const int32_t *ctx;       // [B] tokens in the cache, the chunk included
@@ -616,7 +618,7 @@ struct ExtSplitArgs {
   int32_t B, max_ctx;
 };
 
-template <int D, bool BF16, bool MFMA, int QC>
+template <int D, bool BF16, bool, int QC>
 __global__ void __launch_bounds__(256) attn_ext_split_kernel(KArgs a, ExtSplitArgs x) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -653,7 +655,7 @@ __global__ void __launch_bounds__(256) attn_ext_split_kernel(KArgs a, ExtSplitAr
   sg.j0 = 0;
   sg.j1 = (sg.ctx + kPageSize - 1) / kPageSize;
   sg.nk = sg.nv = nullptr;
-  run_segment<D, BF16, MFMA, QC>(a, sg, lane, true, 0, 1);
+  run_segment<D, BF16, false, QC>(a, sg, lane, true, 0, 1);
 }
 
 template <int D, bool BF16>

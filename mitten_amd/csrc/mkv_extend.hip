@@ -105,7 +105,8 @@ __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, in
   constexpr int TILE = 16 * RB;
   constexpr int BCH = 2 * 16 * CPR;                   // chunks of K + V of one block
   constexpr int NCH = KB * BCH;                       // chunks of one step (KB blocks)
-  constexpr int LPL = (NCH + 64 * W - 1) / (64 * W);  // loads per lane per step
+  constexpr int LPL = NCH / (64 * W);                 // loads per lane per step
+  static_assert(NCH % (64 * W) == 0, "every lane loads the same number of chunks");
   static_assert(R % 2 == 0, "even ring: stage s of an unrolled round uses LDS buffer s & 1");
   __shared__ __attribute__((aligned(16))) uint8_t tiles[2][KB][2][TILE];
   // (Opaque, as the kernel's arguments: no lane offset is kept in registers
@@ -176,12 +177,12 @@ __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, in
 #pragma unroll
     for (int i = 0; i < LPL; i++) {
       const int c = tid + 64 * W * i;
-      const int kb = min(c / BCH, KB - 1), rem = c % BCH;
+      const int kb = c / BCH, rem = c % BCH;
       const int kv = rem / (16 * CPR), rem2 = rem % (16 * CPR), row = rem2 / CPR, cc = rem2 % CPR;
       int32_t bk = blk[0];
 #pragma unroll
       for (int j = 1; j < KB; j++) bk = kb == j ? blk[j] : bk;
-      const bool real = c < NCH && step * KB + kb < n;
+      const bool real = step * KB + kb < n;
       const uint8_t *plane = a.k_plane + (kv ? v_off : 0);
       const int64_t off = real ? (int64_t)bk * a.block_bytes + (int64_t)row * a.row_bytes + h * RB + 16 * cc
                                : spare + 16 * (lane & 7);
@@ -218,19 +219,12 @@ __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, in
     }
   }
   if (__builtin_amdgcn_readfirstlane(__syncthreads_or(slow))) fast_end = st0;
-  // A wave past the step's chunks (head_dim 64 with 16 waves) loads the
-  // step's last chunks again and does not store them: one load form, so the
-  // compiler's in-order load counting stays exact.
-  constexpr bool kAllVal = NCH % (64 * W) == 0;
   uint32_t flo[LPL], fwr[LPL];  // lane offset in the block; LDS offset in one ring buffer
   int fkb[LPL];                 // wave-uniform block of the step
   const uint8_t *fpl[LPL];      // wave-uniform plane (K or V)
-  bool fval[LPL];               // wave-uniform: the wave's chunk is stored
 #pragma unroll
   for (int i = 0; i < LPL; i++) {
-    const int cw = 64 * (wave + W * i);
-    fval[i] = kAllVal || cw < NCH;
-    const int cu = min(cw, NCH - 64);
+    const int cu = 64 * (wave + W * i);
     const int pl = cu / (16 * CPR), kv = pl & 1;
     fkb[i] = pl >> 1;
     fpl[i] = a.k_plane + (kv ? v_off : 0);
@@ -276,37 +270,35 @@ __device__ __forceinline__ void extend_tile(const KArgs &a, const ExtArgs &e, in
 #pragma unroll
     for (int i = 0; i < LPL; i++) {
       if constexpr (FAST) {
-        if (kAllVal || fval[i]) *reinterpret_cast<u32x4 *>(&tiles[s & 1][0][0][0] + fwr[i]) = ring[s][i];
+        *reinterpret_cast<u32x4 *>(&tiles[s & 1][0][0][0] + fwr[i]) = ring[s][i];
         continue;
       }
       const int c = tid + 64 * W * i;
-      if (c < NCH) {
-        const int kb = c / BCH, rem = c % BCH;
-        const int kv = rem / (16 * CPR), rem2 = rem % (16 * CPR), row = rem2 / CPR, cc = rem2 % CPR;
-        // V rows past the context or of a rejected block are stored as
-        // zeros (stale slots may hold any bit pattern, and p = 0 times NaN
-        // would poison O); K rows there are masked in the scores instead.
-        u32x4 val = ring[s][i];
-        const int key = kPageSize * (step * KB + kb) + row;
-        if (kv && (((badr[s] >> kb) & 1) || key >= ctx)) val = u32x4{0u, 0u, 0u, 0u};
-        if (kv && key > qlo_wg) {
-          // Hidden from the tile's first row, with p = 0, and 0 times Inf or
-          // NaN is NaN: such values (exponent of all ones) are left out here
-          // and added to the rows that see them once the tile is done.
-          uint32_t odd = 0;
+      const int kb = c / BCH, rem = c % BCH;
+      const int kv = rem / (16 * CPR), rem2 = rem % (16 * CPR), row = rem2 / CPR, cc = rem2 % CPR;
+      // V rows past the context or of a rejected block are stored as
+      // zeros (stale slots may hold any bit pattern, and p = 0 times NaN
+      // would poison O); K rows there are masked in the scores instead.
+      u32x4 val = ring[s][i];
+      const int key = kPageSize * (step * KB + kb) + row;
+      if (kv && (((badr[s] >> kb) & 1) || key >= ctx)) val = u32x4{0u, 0u, 0u, 0u};
+      if (kv && key > qlo_wg) {
+        // Hidden from the tile's first row, with p = 0, and 0 times Inf or
+        // NaN is NaN: such values (exponent of all ones) are left out here
+        // and added to the rows that see them once the tile is done.
+        uint32_t odd = 0;
 #pragma unroll
-          for (int x = 0; x < 4; x++) odd |= (val[x] & 0x7f807f80u) + 0x00800080u;
-          if (odd & 0x80008000u) {
+        for (int x = 0; x < 4; x++) odd |= (val[x] & 0x7f807f80u) + 0x00800080u;
+        if (odd & 0x80008000u) {
 #pragma unroll
-            for (int x = 0; x < 4; x++) {
-              const uint32_t one = (((val[x] & 0x7f807f80u) + 0x00800080u) >> 15) & 0x00010001u;
-              val[x] &= ~((one << 16) - one);
-            }
-            odd_s = 1;
+          for (int x = 0; x < 4; x++) {
+            const uint32_t one = (((val[x] & 0x7f807f80u) + 0x00800080u) >> 15) & 0x00010001u;
+            val[x] &= ~((one << 16) - one);
           }
+          odd_s = 1;
         }
-        *reinterpret_cast<u32x4 *>(tiles[s & 1][kb][kv] + row * RB + ((cc ^ (kv ? ext_v_swz(row, CPR) : ext_k_swz(row, CPR))) << 4)) = val;
       }
+      *reinterpret_cast<u32x4 *>(tiles[s & 1][kb][kv] + row * RB + ((cc ^ (kv ? ext_v_swz(row, CPR) : ext_k_swz(row, CPR))) << 4)) = val;
     }
     __syncthreads();
     if (!computes) return;
@@ -978,13 +970,14 @@ extern "C" int mkv_extend_attention_host(mkv_pool *pool, int32_t layer, const vo
   return rc ? rc : rr;
 }
 
-// The extend kernel's instantiation for head_dim D and W waves (4, 8 or 16; 8
-// at head_dim 256: 16 waves cap the registers at 128, and its state then
-// spills; 4 waves would carry 8 loads a lane and step).
+// The extend kernel's instantiation for head_dim D and W waves: 4 or 8 at
+// head_dim 64 (16 gained 0.01% over 280 calls, at most 2%), 4, 8 or 16 at 128,
+// 8 at 256 (16 waves cap the registers at 128, and its state then spills; 4
+// waves would carry 8 loads a lane and step).
 const void *mkv::ext_kernel(int D, int W) {
 #define MKV_EXT_FN(DD, WW) reinterpret_cast<const void *>(&attn_extend_kernel<DD, WW, kExtKB, kExtR>)
   switch (D) {
-    case 64: return W == 4 ? MKV_EXT_FN(64, 4) : W == 8 ? MKV_EXT_FN(64, 8) : MKV_EXT_FN(64, 16);
+    case 64: return W == 4 ? MKV_EXT_FN(64, 4) : MKV_EXT_FN(64, 8);
     case 128: return W == 4 ? MKV_EXT_FN(128, 4) : W == 8 ? MKV_EXT_FN(128, 8) : MKV_EXT_FN(128, 16);
     default: return MKV_EXT_FN(256, 8);
   }
@@ -1028,7 +1021,7 @@ struct ExtCost {
   double merge, merge_value;    // the merge launch; a partial value written and read
 };
 static const ExtCost kExtCost[3] = {
-    {{.31, .31, .45}, {.011, .012, .011}, {.13, .19, .016}, .0084, 1.1, 4.6, .83, .44, 2.5, 2.3e-6},
+    {{.31, .31, 0}, {.011, .012, 0}, {.13, .19, 0}, .0084, 1.1, 4.6, .83, .44, 2.5, 2.3e-6},  // 4 and 8 waves
     {{.32, .48, .31}, {.020, .029, .025}, {.18, .16, .18}, .025, 3.6, 5.2, .26, .10, 1.5, 1.8e-6},
     {{0, .68, 0}, {0, .095, 0}, {0, .033, 0}, .019, 4.4, 2.8, .60, .78, 5.9, 1.2e-6},  // 8 waves only
 };
@@ -1074,8 +1067,8 @@ int mkv::launch_ext_tiles(Pool *p, KArgs &a, ExtArgs &e, int split_cap, hipStrea
   const double share = e.causal ? 1.0 - 0.5 * (double)max_q_len / (double)max_ctx_len : 1.0;
   const int cus = device_cus(p);
   const ExtCost &ec = kExtCost[g.D == 64 ? 0 : g.D == 128 ? 1 : 2];
-  // Waves per workgroup (8 at head_dim 256, at most 8 beside a decode launch;
-  // waves past the tile's rows share the loads), row waves per tile (half of
+  // Waves per workgroup (ext_kernel's, at most 8 beside a decode launch; waves
+  // past the tile's rows share the loads), row waves per tile (half of
   // them or more, or what the rows fill) and key-range splits: the least cost.
   // A key range splits only where the launch leaves resident slots empty (short
   // chunks over long contexts), in at most split_cap of at least 8 steps apiece
@@ -1086,12 +1079,13 @@ int mkv::launch_ext_tiles(Pool *p, KArgs &a, ExtArgs &e, int split_cap, hipStrea
   // one much (14 heads on 2 of 64, 40 short prompts beside one chunk after 8k:
   // 112 us without, 65 with).
   int W = 0;
+  const int most_waves = g.D == 128 && !beside ? 16 : 8;
   auto choose = [&](int cap) {
-    W = g.D == 256 ? 8 : row_waves_max <= 4 ? 4 : row_waves_max <= 8 || beside ? 8 : 16;
+    W = g.D == 256 ? 8 : row_waves_max <= 4 ? 4 : row_waves_max <= 8 ? 8 : most_waves;
     e.splits = 1;
     e.row_waves = (int32_t)std::min<int64_t>(W, row_waves_max);
     double best = INFINITY;
-    for (int w = g.D == 256 ? 8 : 4; w <= (beside || g.D == 256 ? 8 : 16); w *= 2) {
+    for (int w = g.D == 256 ? 8 : 4; w <= most_waves; w *= 2) {
       if (g.D < 256 && w > 4 && row_waves_max < w / 4) break;
       // Resident workgroups per CU of this instantiation (occupancy query, once
       // per pool); one beside a decode launch.

@@ -25,8 +25,8 @@ SHAPES = {
     "llama8b": (32, 8, 128),
     "g16": (64, 4, 128),
     "mha": (4, 4, 64),
-    "d256-g4": (16, 4, 256),   # head_dim 256 with 4 waves per workgroup
-    "d256-g16": (16, 1, 256),  # head_dim 256 with 16 waves per workgroup
+    "d256-g4": (16, 4, 256),
+    "d256-g16": (16, 1, 256),
 }
 # Shapes beside the engine's bf16 ones: f32, head_dim 32, large groups.
 SEGMENT_SHAPES = {
@@ -90,7 +90,7 @@ def test_extend_attention_zero_sink():
 
 @pytest.mark.parametrize("shape", ["qwen7b", "qwen0.5b", "mha"])
 def test_extend_short_chunks(shape):
-    """Chunks of at most 16 tokens (one query sub-tile per workgroup) after
+    """Chunks of at most 16 tokens (workgroups that compute few rows) after
     prefixes of assorted lengths."""
     got, ref, dec, q_indptr = _case(shape, [16, 300, 1000, 47, 8], [16, 1, 9, 16, 3], 97)
     assert_attention_close(got, ref, "bf16")
@@ -160,8 +160,8 @@ def test_extend_split_key_ranges_with_empty_splits():
 
 
 def test_extend_split_rejects_chunk_past_max_q_len():
-    """With split key ranges a chunk longer than max_q_len is reported
-    (its partial rows would lie past the workspace), not written."""
+    """With split key ranges chunks past num_seqs * max_q_len tokens are
+    reported (their partial rows would lie past the workspace), not written."""
     Hq, Hkv, D = SHAPES["qwen7b"]
     rng = wl.SplitMix64(99)
     batch = wl.decode_batch_from_contexts([2000 - 1], rng, extra_blocks=2)
@@ -355,3 +355,52 @@ def test_extend_captured_before_the_workspace_has_room():
             pool.extend_attention(0, *args, out=eager)
             assert_attention_close(to_host(eager), ref, "bf16")
         pool.check()
+
+
+@pytest.mark.parametrize("shape", [(28, 4, 128, "bf16"), (12, 1, 64, "bf16"), (40, 2, 256, "bf16"), (18, 1, 32, "bf16"),
+                                   (14, 2, 64, "f32"), (4, 4, 128, "f32"), (9, 1, 256, "f32"), (20, 2, 32, "f32")])
+def test_extend_segments(shape):
+    """Per-token decode segments, which the C ABI's FORCE_VALU flag selects at
+    every head_dim (head_dim 32 has no other path), with groups of more than
+    one chunk of 8 query heads."""
+    Hq, Hkv, D, dt = shape
+    ctx, nq = [1, 17, 40, 300, 97], [1, 17, 25, 64, 1]
+    batch = wl.decode_batch_from_contexts([c - 1 for c in ctx], wl.SplitMix64(114), extra_blocks=2)
+    desc = PoolDesc(1, Hkv, Hq, D, batch.num_blocks, dt)
+    host = normal(115, desc.shape, dt)
+    q_indptr = np.concatenate([[0], np.cumsum(nq)]).astype(np.int32)
+    q = normal(116, (int(q_indptr[-1]), Hq, D), dt)
+    with DeviceKvPool(desc) as pool:
+        pool.write(host)
+        qd = to_device(q)
+        out = to_device(np.zeros_like(q))
+        meta = [_i32(a) for a in (q_indptr, batch.block_indptr, batch.block_ids, batch.ctx_lens)]
+        dp._raise(pool._lib.mkv_extend_attention(
+            pool._h, 0, dp._dptr(qd), dp._dptr(out), *[dp._dptr(t) for t in meta], len(ctx), max(nq), max(ctx),
+            float(np.float32(D ** -0.5)), dp.ATTN_FORCE_VALU, dp._stream_handle(None)))
+        pool.check()
+        got = to_host(out)
+    ref = orc.extend_attention(odesc(desc), host, 0, widen(q), q_indptr, batch.block_indptr, batch.block_ids,
+                               batch.ctx_lens)
+    assert_attention_close(got, ref, dt)
+
+
+@pytest.mark.parametrize("shape,num_seqs,chunk", [
+    # the waves per workgroup and key-range splits that a device of 256 CUs
+    # takes where the other tests' sizes take four waves
+    ((14, 2, 64), 64, (48, 48)),    # 8 waves, unsplit
+    ((16, 1, 64), 100, (5, 1000)),  # 8 waves, split
+    ((8, 8, 128), 100, (20, 20)),   # 8 waves, unsplit
+    ((16, 1, 128), 100, (5, 2500)), # 8 waves, split
+    ((8, 4, 128), 48, (48, 48)),    # 16 waves, unsplit
+    ((16, 1, 128), 48, (5, 1000)),  # 16 waves, split
+])
+def test_extend_row_tiles_in_wide_batches(shape, num_seqs, chunk):
+    """Batches that fill the device: one chunk of the given new tokens and
+    context among chunks of one to five tokens."""
+    nq = [1 + b % min(5, chunk[0]) for b in range(num_seqs)]
+    ctx = [n + 7 * b % 40 for b, n in enumerate(nq)]
+    nq[num_seqs // 2], ctx[num_seqs // 2] = chunk
+    got, ref, dec, q_indptr = _case(shape, ctx, nq, 117)
+    assert_attention_close(got, ref, "bf16")
+    assert_attention_close(dec, ref[q_indptr[1:] - 1], "bf16")
