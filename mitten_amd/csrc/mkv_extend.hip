@@ -590,13 +590,14 @@ attn_extend_kernel(KArgs, ExtArgs) {
 // in the loop; at head_dim 64 the next block's loads are issued before
 // this one is used.
 //
-// What bounds it: short prompts (8 of 32-512 tokens, 14 query heads, 36.7 us a
-// layer) by the serial chain of a tile, 30% of the f32 matrix rate; long ones
-// by the matrix cores and the softmax between them (8 x 512: 51 TFLOP/s, 64 x
-// 512 after 2,000: 108 of 157). One decode segment per query token, which
-// every f32 prompt took before, read the context once per token: 139 us for
-// the same short prompts. Eight waves per tile: 48.8 us; one 16-row group per
-// workgroup: 37.1 us, and 58 for 102 TFLOP/s at 64 x 512 after 2,000.
+// What bounds it: short prompts (8 of 32-512 tokens, 14 query heads, 38 us a
+// layer) by the serial chain of a tile, the matrix cores busy 27% of the time;
+// long ones by the matrix cores and the softmax between them (8 x 512: 62
+// TFLOP/s, 64 x 512 after 2,000: 106 of 157). One decode segment per query
+// token, which every f32 prompt took before, read the context once per token:
+// 139 us for the same short prompts. When it was written, at 36.7 us: eight
+// waves per tile 48.8 us; one 16-row group per workgroup 37.1 us, and 58 for
+// 102 TFLOP/s at 64 x 512 after 2,000.
 //
 // All in f32 on v_mfma_f32_16x16x4 (twice the rate of unpacked f32 FMAs, and
 // no cross-lane score sums). Lane = (g = lane / 16, c = lane % 16):
